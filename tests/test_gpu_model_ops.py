@@ -120,6 +120,38 @@ def test_silu_mul_matches_torch(rows, inter):
     assert ulps(out, want) <= 1
 
 
+def _off(t, elems):
+    """A copy of rows t at an offset of `elems` from an aligned start, rows `elems` longer."""
+    rows, cols = t.shape
+    buf = torch.zeros((rows, cols + elems), dtype=t.dtype, device=t.device)
+    buf[:, elems:] = t
+    return buf[:, elems:]
+
+
+@pytest.mark.parametrize("rows,hq,hkv,d", [(1, 1, 1, 16), (70, 3, 1, 48), (130, 14, 2, 64),
+                                           (65, 12, 2, 128), (3, 2, 1, 512), (2, 2, 1, 24)])
+def test_rope_row_and_element_forms_agree(rows, hq, hkv, d):
+    """The workgroup-per-row form against the element form (taken for the same rows one
+    element off alignment): the same operations in the same order, so bit-identical."""
+    qkv = randn(rows, (hq + 2 * hkv) * d, seed=21)
+    positions = torch.randint(0, 40000, (rows,), generator=gen(22), device=DEV)
+    inv_freq = 1.0 / 1e6 ** (torch.arange(0, d, 2, device=DEV, dtype=torch.float32) / d)
+    want = ops.rope_qkv(_off(qkv, 1), positions, inv_freq, hq, hkv, d)
+    for src in (qkv, _off(qkv, 8)):
+        for got, w in zip(ops.rope_qkv(src, positions, inv_freq, hq, hkv, d), want):
+            assert torch.equal(got, w)
+
+
+@pytest.mark.parametrize("rows,inter", [(1, 8), (3, 2040), (67, 2056), (5, 20), (70000, 8)])
+def test_silu_vector_and_element_forms_agree(rows, inter):
+    """Bit-identical, infinities and NaN included (inter 20 has the element form only)."""
+    gu = randn(rows, 2 * inter, seed=23, scale=3.0)
+    gu[0, 0], gu[0, 1], gu[0, inter + 2], gu[0, 3] = float("inf"), float("-inf"), float("nan"), 88.0
+    want = ops.silu_mul(_off(gu, 1))
+    for src in (gu, _off(gu, 8)):
+        assert torch.equal(ops.silu_mul(src).view(torch.int16), want.view(torch.int16))
+
+
 @pytest.mark.parametrize("m,n,k", [(1, 2048, 1536), (3, 1536, 8960), (8, 17920, 1536),
                                    (16, 1000, 96), (17, 300, 1536), (32, 151936, 1536)])
 def test_gemm_skinny_matches_fp32_product(m, n, k):
