@@ -68,6 +68,23 @@ def context_lens_from_positions(positions: torch.Tensor, active_mask: torch.Tens
         torch.int32)
 
 
+def decode_step_inputs(block_tables: torch.Tensor, positions: torch.Tensor,
+                       active_mask: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor]:
+    """(int32 tables, int32 context lengths) of a batched decode call: one launch for the
+    contract's dense GPU tensors (int64 positions, float32 or bool mask), tensor by tensor
+    for any other type, stride or device."""
+    if not ops.decode_inputs_supported(positions, active_mask):
+        tables = block_tables if block_tables.dtype == torch.int32 else block_tables.to(torch.int32)
+        return tables, context_lens_from_positions(positions, active_mask)
+    if block_tables.dtype == torch.int64 and block_tables.is_contiguous() and \
+            block_tables.ndim == 2 and block_tables.shape[0] == positions.numel() and \
+            block_tables.device == positions.device:
+        ctx, tables = ops.decode_inputs(positions, active_mask, block_tables)
+        return tables, ctx
+    tables = block_tables if block_tables.dtype == torch.int32 else block_tables.to(torch.int32)
+    return tables, ops.decode_inputs(positions, active_mask)[0]
+
+
 def paged_decode_batch(q: torch.Tensor, cache, layer: int, block_tables: torch.Tensor,
                        positions: torch.Tensor, active_mask: torch.Tensor, *,
                        k_new: torch.Tensor | None = None,
@@ -83,8 +100,7 @@ def paged_decode_batch(q: torch.Tensor, cache, layer: int, block_tables: torch.T
         raise ValueError("invalid static decode inputs")
     if q.shape[1] % cache.layout.kv_heads:
         raise ValueError("Q heads must be a multiple of KV heads")
-    ctx = context_lens_from_positions(positions, active_mask)
-    tables = block_tables if block_tables.dtype == torch.int32 else block_tables.to(torch.int32)
+    tables, ctx = decode_step_inputs(block_tables, positions, active_mask)
     return ops.paged_decode(q, cache.k[layer], cache.v[layer], tables, ctx,
                             scale=1.0 / math.sqrt(q.shape[-1]), k_new=k_new, v_new=v_new)
 

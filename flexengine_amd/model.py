@@ -207,8 +207,7 @@ class Qwen2Model:
         active = active_mask.reshape(-1)
         # the batched backend contract's conversions, once per step for all layers
         # (paged_attention.py:115,131,138): length = position + 1, 0 for inactive rows
-        ctx = attention.context_lens_from_positions(positions, active)
-        tables = block_tables if block_tables.dtype == torch.int32 else block_tables.to(torch.int32)
+        tables, ctx = attention.decode_step_inputs(block_tables, positions, active)
         tables = tables.contiguous()
         # the decode plan (split-K partition and block rows) of this step, shared by
         # every layer: the tables and lengths are the same for all of them

@@ -150,6 +150,40 @@ def gather_tables(mirror: torch.Tensor, row_len: torch.Tensor, rows: torch.Tenso
     return out
 
 
+_MASK_BYTES = {torch.float32: 4, torch.bool: 1, torch.uint8: 1}
+
+
+def decode_inputs_supported(positions: torch.Tensor, active_mask: torch.Tensor) -> bool:
+    """Whether decode_inputs takes these tensors as they are: dense int64 positions and a
+    dense float32 / bool / uint8 mask of as many elements, on one GPU."""
+    return (positions.device.type == "cuda" and active_mask.device == positions.device
+            and positions.dtype == torch.int64 and active_mask.dtype in _MASK_BYTES
+            and positions.is_contiguous() and active_mask.is_contiguous()
+            and active_mask.numel() == positions.numel())
+
+
+def decode_inputs(positions: torch.Tensor, active_mask: torch.Tensor,
+                  block_tables: torch.Tensor | None = None
+                  ) -> tuple[torch.Tensor, torch.Tensor | None]:
+    """(int32 context lengths, int32 tables) of the batched decode contract in one launch
+    (fe_decode_inputs); block_tables, if given, dense int64 [B, W]."""
+    if not decode_inputs_supported(positions, active_mask):
+        raise ValueError("positions must be dense int64 and the mask dense float32, bool or uint8")
+    dev = _require_gpu(positions, active_mask, block_tables)
+    batch, width, tables = positions.numel(), 0, None
+    if block_tables is not None:
+        if block_tables.ndim != 2 or block_tables.shape[0] != batch or \
+                block_tables.dtype != torch.int64 or not block_tables.is_contiguous():
+            raise ValueError("block_tables must be dense int64 [batch, W]")
+        width = block_tables.shape[1]
+        tables = torch.empty((batch, width), dtype=torch.int32, device=dev)
+    lens = torch.empty((batch,), dtype=torch.int32, device=dev)
+    _lib.call("fe_decode_inputs", positions.data_ptr(), active_mask.data_ptr(),
+              _MASK_BYTES[active_mask.dtype], _ptr(block_tables), batch, width, lens.data_ptr(),
+              _ptr(tables), _stream(dev))
+    return lens, tables
+
+
 def write_kv_decode(k_new: torch.Tensor, v_new: torch.Tensor, k_pool: torch.Tensor,
                     v_pool: torch.Tensor, block_tables: torch.Tensor,
                     context_lens: torch.Tensor) -> None:

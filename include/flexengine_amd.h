@@ -162,6 +162,19 @@ int fe_gather_tables(const int32_t* mirror, int mirror_stride, const int32_t* ro
                      int pad_block, int32_t* out, int out_stride, fe_stream_t stream);
 
 /*
+ * The batched decode contract's conversions in one launch: for b < batch,
+ *   lens_out[b] = (int32)(positions[b] + 1) if active_mask[b] != 0, else 0,
+ * and, unless block_tables is NULL, tables_out[b, j] = (int32)block_tables[b, j]
+ * for j < width (both dense).  positions and block_tables are int64; active_mask
+ * holds 4-byte floats (mask_bytes 4; NaN is active) or bytes (mask_bytes 1).
+ * Replaces the per-call conversions of the batched decode callers
+ * (src/flexengine/inference/kernels/paged_attention.py:115,131,138).
+ */
+int fe_decode_inputs(const int64_t* positions, const void* active_mask, int mask_bytes,
+                     const int64_t* block_tables, int batch, int width, int32_t* lens_out,
+                     int32_t* tables_out, fe_stream_t stream);
+
+/*
  * Block-table gather ("materialize"): for every sequence b and position
  * t < context_lens[b],
  *   k_out[out_offsets[b] + t] = k_pool[block_tables[b, t/bs], t%bs]   (and v)

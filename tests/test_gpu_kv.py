@@ -233,3 +233,25 @@ def test_graph_inputs_pad_rows_with_a_scratch_block():
         assert inp["block_tables"][row].tolist() == [scratch] * 4
     with pytest.raises(ValueError):
         step.graph_inputs([Chunk("a", [1], 0)] * 5, 4)
+
+
+@pytest.mark.parametrize("batch,width", [(1, 1), (8, 32), (64, 257), (300, 3)])
+@pytest.mark.parametrize("mask_dtype", [torch.float32, torch.bool, torch.uint8, torch.int64])
+def test_decode_step_inputs_match_the_tensor_route(batch, width, mask_dtype):
+    """The one-launch conversion against the general one, over every form the dispatch
+    tells apart: mask types, int32 / int64 / strided tables, strided positions, NaN masks."""
+    from flexengine_amd import attention
+    g = torch.Generator(device=DEV).manual_seed(batch)
+    pos = torch.randint(0, 1 << 20, (batch,), generator=g, device=DEV)
+    pos[0] = 2 ** 31 + 5                      # wraps like .to(torch.int32)
+    mask = (torch.rand(batch, generator=g, device=DEV) < 0.6).to(mask_dtype)
+    if mask_dtype == torch.float32:
+        mask[-1] = float("nan")               # nan != 0: active
+    tables = torch.randint(0, 1 << 30, (batch, width), generator=g, device=DEV)
+    want_ctx = attention.context_lens_from_positions(pos, mask)
+    wide = torch.stack([tables, tables], -1)[..., 0]          # strided
+    for t in (tables, tables.int(), wide):
+        for p in (pos, torch.stack([pos, pos], -1)[:, 0]):
+            got_t, got_ctx = attention.decode_step_inputs(t, p, mask)
+            assert got_t.dtype == got_ctx.dtype == torch.int32
+            assert torch.equal(got_t, tables.int()) and torch.equal(got_ctx, want_ctx)
