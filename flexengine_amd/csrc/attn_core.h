@@ -232,40 +232,54 @@ struct TileCore {
   }
 };
 
-// fp32 tile engine (pools, q and output in fp32), in the 16-bit engines'
-// register layout, so the decode kernel around it -- the cross-wave combine,
-// the split-K partials and their merge -- is the same:
+// fp32 tile engine (pools, q and output in fp32) for RT 16-column row tiles, near the
+// 16-bit engines' register layout, so the decode kernel around it -- the cross-wave
+// combine, the split-K partials and their merge -- is the same:
 //   S^T = K . Q^T on v_mfma_f32_16x16x4_f32: lane (g,n) loads dims 16c+4g .. +3
 //     of key n and of column n's query (one 16-byte load per chunk c); MFMA
 //     (c, j) contracts dim 16c + 4g + j in k-slot g.  -> lane (g,n) holds the
 //     scores of column n for keys 4g..4g+3.
-//   O^T += V^T . P^T, MFMA r taking keys 4g + r in k-slot g: A = V[key 4g+r]
-//     [dim 16x+n] (a dword per (r, x); the 16 lanes of a group read a 64-byte
-//     run of one row), B = the lane's probability of key 4g + r.  -> lane (g,n)
-//     accumulates O[col n][16x + 4g + i].
+//   O^T += V^T . P^T, MFMA (w, j, r) taking keys 4g + r in k-slot g: A = V[key 4g+r]
+//     [dim 64w + 4n + j] (one 16-byte load per (r, 64-dim group w); the 16 lanes of a
+//     group read 256 consecutive bytes of a row), B = the lane's probability of key
+//     4g + r.  -> lane (g,n) accumulates O[col n][64w + 4(4g + i) + j] in o[4w + j][i];
+//     finish() turns each 4x4 of registers, so that o[x] then holds the 4 consecutive
+//     dims from f32_dim0(x, g).
 // Probabilities stay fp32; the online softmax is the 16-bit engines' (base 2,
 // the same rescale slack).  Any block size: a table lookup per key row, or
 // (LIST, block sizes that are multiples of 16) the wave's tile rows held one
-// per lane.  Column n accepts keys < limit (decode: tok_end; prefill: its
-// position + 1).
+// per lane.  Column n of row tile rt accepts keys < limit[rt] (decode: tok_end;
+// prefill: its position + 1).
+//
+// What bounds it: 64 MFMAs of 32 cycles per 16-key tile and row tile at D = 128
+// against 16 KB of loads.  The tile loads are raw buffer loads through one scalar
+// descriptor per tile with loop-invariant lane offsets (rows past the extent read as
+// zeros): 8 + 8 loads and no per-row addresses.  With a dword load per V element, 64-bit
+// row addresses and a select per element the engine held 304 VGPRs, one wave per SIMD,
+// and a tile took 3190 cycles; it now fits two (decode) or three (prefill) waves.
 //
 // PAD: the real head_dim dr is below D (a multiple of 4): rows are dr floats
 // apart within a pool row, the dims past dr are zeros in K and V (not loaded,
 // and not written by the page write), and q is zero there too.
-template <int D, bool LIST = false, bool PAD = false>
+__device__ __forceinline__ constexpr int f32_dim0(int x, int g) {
+  return 64 * (x >> 2) + 16 * g + 4 * (x & 3);
+}
+
+template <int D, bool LIST = false, bool PAD = false, int RT = 1>
 struct F32Core {
   static constexpr int NC = D / 16;  // 16-byte K and q chunks per lane
+  static constexpr int NW = D / 64;  // 64-dim groups of V
   static constexpr int NX = D / 16;  // output tiles of 16 dims
 
   const float* k_pool;
   const float* v_pool;
   const int32_t* trow;  // block-table row of the sequence
-  int64_t rs;           // elements per pool row (kv_heads * head_dim)
+  int64_t rs;           // elements per pool row (kv_heads * head_dim; LIST: 64 rs < 2^31)
   int hoff;             // kv_head * head_dim
   int dr;               // PAD: the real head_dim
   int W, NB, BS, bs_log2;
   int tok_end;          // keys >= tok_end are never read
-  int limit;            // this lane's column accepts keys < limit
+  int limit[RT];        // this lane's column of each row tile accepts keys < limit
   float scale_log2;
   // optional fused page write of the decode token (position new_pos)
   const float* knew_row;
@@ -280,10 +294,10 @@ struct F32Core {
   int t_first, step;
   int row_vec, list_base;
 
-  f32x4 qv[NC];
-  float m_run;
-  float l_run;
-  f32x4 o[NX];
+  f32x4 qv[RT][NC];
+  float m_run[RT];
+  float l_run[RT];
+  f32x4 o[RT][NX];
 
   __device__ __forceinline__ int64_t pool_row(int tok) const {
     int page = tok >> bs_log2;
@@ -296,137 +310,252 @@ struct F32Core {
     list_base = k0;
     row_vec = (int)pool_row((t_first + (k0 + lane_id()) * step) * kTile);
   }
-  // Pool row of key t0 + r of the wave's k-th tile (key clamped below tok_end).
-  __device__ __forceinline__ int64_t key_row(int k, int t0, int r) const {
-    const int tok = t0 + r < tok_end ? t0 + r : tok_end - 1;
-    if constexpr (LIST)
-      return (int64_t)__builtin_amdgcn_readlane(row_vec, k - list_base) + (tok - t0);
-    else
-      return pool_row(tok);
+  // LIST: descriptor of tile k of a pool, from its first key's row to the end of its
+  // last valid key's row (loads past it return zeros)
+  __device__ __forceinline__ __amdgpu_buffer_rsrc_t tile_rsrc(const float* pool, int k,
+                                                             int t0) const {
+    const int64_t base = (int64_t)__builtin_amdgcn_readlane(row_vec, k - list_base) * rs + hoff;
+    const uint64_t addr = reinterpret_cast<uint64_t>(pool + base);
+    const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)addr);
+    const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(addr >> 32));
+    const int rows = tok_end - t0 < kTile ? tok_end - t0 : kTile;
+    const int nrec = __builtin_amdgcn_readfirstlane(
+        ((rows - 1) * (int)rs + (PAD ? dr : D)) * (int)sizeof(float));
+    return __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<void*>(((uint64_t)hi << 32) | lo), 0,
+                                             nrec, 0x00020000);
   }
 
   __device__ __forceinline__ void init_acc() {
-    m_run = kNegInf;
-    l_run = 0.f;
 #pragma unroll
-    for (int x = 0; x < NX; ++x) o[x] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int rt = 0; rt < RT; ++rt) {
+      m_run[rt] = kNegInf;
+      l_run[rt] = 0.f;
+#pragma unroll
+      for (int x = 0; x < NX; ++x) o[rt][x] = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
   }
 
-  __device__ __forceinline__ void load_tile(int k, f32x4 (&kk)[NC], float (&vv)[4][NX]) {
+  // K of tile k: chunk c of key n.  Fills the tile list when tile k is past it, so it
+  // runs before load_v of the same tile.
+  __device__ __forceinline__ void load_k(int k, f32x4 (&kk)[NC]) {
     const int lane = lane_id();
     const int g = lane >> 4;
     const int n = lane & 15;
+    const int t0 = (t_first + k * step) * kTile;
     if constexpr (LIST) {
       if (k - list_base >= kWave) fill_list(k);  // wave-uniform
-    }
-    const int t0 = (t_first + k * step) * kTile;
-    {
-      const int tk = t0 + n;
-      const int64_t off = key_row(k, t0, n) * rs + hoff + 4 * g;
-      if (tk == new_pos) {
+      const __amdgpu_buffer_rsrc_t r = tile_rsrc(k_pool, k, t0);
+      const uint32_t off = (uint32_t)((n * (int)rs + 4 * g) * (int)sizeof(float));
 #pragma unroll
-        for (int c = 0; c < NC; ++c) {
-          kk[c] = f32x4{0.f, 0.f, 0.f, 0.f};
-          if (!PAD || 16 * c + 4 * g < dr) {
-            kk[c] = *reinterpret_cast<const f32x4*>(knew_row + 16 * c + 4 * g);
-            *reinterpret_cast<f32x4*>(k_pool_w + off + 16 * c) = kk[c];
-          }
-        }
-      } else {
+      for (int c = 0; c < NC; ++c) {
+        if constexpr (PAD) kk[c] = f32x4{0.f, 0.f, 0.f, 0.f};
+        if (!PAD || 16 * c + 4 * g < dr)
+          kk[c] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(r, off + 64 * c, 0, 0));
+      }
+    } else {
+      const int tok = t0 + n < tok_end ? t0 + n : tok_end - 1;
+      const float* row = k_pool + pool_row(tok) * rs + hoff + 4 * g;
 #pragma unroll
-        for (int c = 0; c < NC; ++c) {
-          kk[c] = f32x4{0.f, 0.f, 0.f, 0.f};
-          if (!PAD || 16 * c + 4 * g < dr)
-            kk[c] = *reinterpret_cast<const f32x4*>(k_pool + off + 16 * c);
-        }
+      for (int c = 0; c < NC; ++c) {
+        kk[c] = f32x4{0.f, 0.f, 0.f, 0.f};
+        if (!PAD || 16 * c + 4 * g < dr) kk[c] = *reinterpret_cast<const f32x4*>(row + 16 * c);
       }
     }
+    if (new_pos >= t0 && new_pos < t0 + kTile && t0 + n == new_pos) {
+      float* row = k_pool_w + pool_row(new_pos) * rs + hoff + 4 * g;
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int tv = t0 + 4 * g + r;
-      const bool ok = tv < tok_end;
-      const int64_t off = key_row(k, t0, 4 * g + r) * rs + hoff + n;
-      if (tv == new_pos) {
-#pragma unroll
-        for (int x = 0; x < NX; ++x) {
-          vv[r][x] = 0.f;
-          if (!PAD || 16 * x + n < dr) {
-            vv[r][x] = vnew_row[16 * x + n];
-            v_pool_w[off + 16 * x] = vv[r][x];
-          }
+      for (int c = 0; c < NC; ++c)
+        if (!PAD || 16 * c + 4 * g < dr) {
+          kk[c] = *reinterpret_cast<const f32x4*>(knew_row + 16 * c + 4 * g);
+          *reinterpret_cast<f32x4*>(row + 16 * c) = kk[c];
         }
-      } else {
-#pragma unroll
-        for (int x = 0; x < NX; ++x) {
-          float val = 0.f;
-          if (!PAD || 16 * x + n < dr) val = v_pool[off + 16 * x];
-          vv[r][x] = ok ? val : 0.f;
-        }
-      }
     }
   }
 
-  __device__ __forceinline__ void compute_tile(int k, const f32x4 (&kk)[NC],
-                                               const float (&vv)[4][NX]) {
+  // V of tile k: dims 64w + 4n .. +3 of key 4g + r (zeros for keys past tok_end).
+  __device__ __forceinline__ void load_v(int k, f32x4 (&vv)[4][NW]) {
     const int lane = lane_id();
     const int g = lane >> 4;
+    const int n = lane & 15;
     const int t0 = (t_first + k * step) * kTile;
-    f32x4 sacc = {0.f, 0.f, 0.f, 0.f};
+    if constexpr (LIST) {
+      const __amdgpu_buffer_rsrc_t b = tile_rsrc(v_pool, k, t0);
+      const uint32_t off = (uint32_t)((4 * g * (int)rs + 4 * n) * (int)sizeof(float));
 #pragma unroll
-    for (int c = 0; c < NC; ++c)
+      for (int r = 0; r < 4; ++r)
 #pragma unroll
-      for (int j = 0; j < 4; ++j) sacc = mfma4_f32(kk[c][j], qv[c][j], sacc);
-    float sv[4];
+        for (int w = 0; w < NW; ++w) {
+          if constexpr (PAD) vv[r][w] = f32x4{0.f, 0.f, 0.f, 0.f};
+          if (!PAD || 64 * w + 4 * n < dr)
+            vv[r][w] = __builtin_bit_cast(
+                f32x4, __builtin_amdgcn_raw_buffer_load_b128(
+                           b, off + 256 * w, (uint32_t)(r * (int)rs * (int)sizeof(float)), 0));
+        }
+    } else {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int tok = t0 + 4 * g + i;
-      sv[i] = tok < limit ? sacc[i] * scale_log2 : kNegInf;
+      for (int r = 0; r < 4; ++r) {
+        const int tv = t0 + 4 * g + r;
+        const bool ok = tv < tok_end;
+        const float* row = v_pool + pool_row(ok ? tv : tok_end - 1) * rs + hoff + 4 * n;
+#pragma unroll
+        for (int w = 0; w < NW; ++w) {
+          f32x4 val = f32x4{0.f, 0.f, 0.f, 0.f};
+          if (!PAD || 64 * w + 4 * n < dr) val = *reinterpret_cast<const f32x4*>(row + 64 * w);
+          vv[r][w] = ok ? val : f32x4{0.f, 0.f, 0.f, 0.f};
+        }
+      }
     }
-    float mx = fmaxf(fmaxf(sv[0], sv[1]), fmaxf(sv[2], sv[3]));
-    mx = fmaxf(mx, shfl_xor_f(mx, 16));
-    mx = fmaxf(mx, shfl_xor_f(mx, 32));
-    if (__ballot(mx > m_run + kRescaleSlack)) {  // wave-uniform
-      const float m_new = fmaxf(m_run, mx);
-      const float alpha = m_new == kNegInf ? 1.f : exp2_fast(m_run - m_new);
-      l_run *= alpha;
+    if (new_pos >= t0 && new_pos < t0 + kTile) {  // wave-uniform
 #pragma unroll
-      for (int x = 0; x < NX; ++x) o[x] *= alpha;
-      m_run = m_new;
+      for (int r = 0; r < 4; ++r) {
+        if (t0 + 4 * g + r != new_pos) continue;
+        float* row = v_pool_w + pool_row(new_pos) * rs + hoff + 4 * n;
+#pragma unroll
+        for (int w = 0; w < NW; ++w)
+          if (!PAD || 64 * w + 4 * n < dr) {
+            vv[r][w] = *reinterpret_cast<const f32x4*>(vnew_row + 64 * w + 4 * n);
+            *reinterpret_cast<f32x4*>(row + 64 * w) = vv[r][w];
+          }
+      }
     }
-    const float m_use = m_run == kNegInf ? 0.f : m_run;
-    float p[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) p[i] = exp2_fast(sv[i] - m_use);
-    l_run += (p[0] + p[1]) + (p[2] + p[3]);
-#pragma unroll
-    for (int x = 0; x < NX; ++x)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) o[x] = mfma4_f32(vv[r][x], p[r], o[x]);
   }
 
-  // The wave's tiles t_first, t_first + step, ... below t_end, one tile of
-  // prefetch: while tile k is computed, the loads of tile k + 1 are in flight.
-  __device__ __forceinline__ void run(int first, int stride, int t_end) {
+  // Scores of tile k's keys, then the online softmax: p[rt] = this lane's probabilities
+  // (keys 4g .. 4g+3).  The dims are summed in two chains, so that no MFMA waits for
+  // the one before it.
+  __device__ __forceinline__ void scores(const f32x4 (&kk)[NC], f32x4 (&sacc)[RT]) const {
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt) {
+      f32x4 s0 = {0.f, 0.f, 0.f, 0.f}, s1 = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int c = 0; c < NC; c += 2)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          s0 = mfma4_f32(kk[c][j], qv[rt][c][j], s0);
+          s1 = mfma4_f32(kk[c + 1][j], qv[rt][c + 1][j], s1);
+        }
+      sacc[rt] = s0 + s1;
+    }
+  }
+  __device__ __forceinline__ void softmax(int k, const f32x4 (&sacc)[RT], f32x4 (&p)[RT]) {
+    const int g = lane_id() >> 4;
+    const int t0 = (t_first + k * step) * kTile;
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt) {
+      float sv[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        sv[i] = t0 + 4 * g + i < limit[rt] ? sacc[rt][i] * scale_log2 : kNegInf;
+      float mx = fmaxf(fmaxf(sv[0], sv[1]), fmaxf(sv[2], sv[3]));
+      mx = fmaxf(mx, shfl_xor_f(mx, 16));
+      mx = fmaxf(mx, shfl_xor_f(mx, 32));
+      if (__ballot(mx > m_run[rt] + kRescaleSlack)) {  // wave-uniform
+        const float m_new = fmaxf(m_run[rt], mx);
+        const float alpha = m_new == kNegInf ? 1.f : exp2_fast(m_run[rt] - m_new);
+        l_run[rt] *= alpha;
+#pragma unroll
+        for (int x = 0; x < NX; ++x) o[rt][x] *= alpha;
+        m_run[rt] = m_new;
+      }
+      const float m_use = m_run[rt] == kNegInf ? 0.f : m_run[rt];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) p[rt][i] = exp2_fast(sv[i] - m_use);
+      l_run[rt] += (p[rt][0] + p[rt][1]) + (p[rt][2] + p[rt][3]);
+    }
+  }
+  __device__ __forceinline__ void pv(const f32x4 (&vv)[4][NW], const f32x4 (&p)[RT]) {
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+#pragma unroll
+      for (int w = 0; w < NW; ++w)
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+          for (int rt = 0; rt < RT; ++rt)
+            o[rt][4 * w + j] = mfma4_f32(vv[r][w][j], p[rt][r], o[rt][4 * w + j]);
+  }
+  __device__ __forceinline__ void compute_tile(int k, const f32x4 (&kk)[NC],
+                                               const f32x4 (&vv)[4][NW]) {
+    f32x4 sacc[RT], p[RT];
+    scores(kk, sacc);
+    softmax(k, sacc, p);
+    pv(vv, p);
+  }
+
+  __device__ __forceinline__ int begin(int first, int stride, int t_end) {
     t_first = first;
     step = stride;
     const int ntiles = first < t_end ? (t_end - first + stride - 1) / stride : 0;
+    if constexpr (LIST) {
+      if (ntiles > 0) fill_list(0);
+    }
+    return ntiles;
+  }
+
+  // The wave's tiles t_first, t_first + step, ... below t_end, a whole tile of
+  // prefetch (HBM-bound callers): while tile k is computed, the loads of tile k + 1
+  // are in flight.
+  __device__ __forceinline__ void run(int first, int stride, int t_end) {
+    const int ntiles = begin(first, stride, t_end);
     if (ntiles == 0) return;
-    if constexpr (LIST) fill_list(0);
     f32x4 ka[NC], kb[NC];
-    float va[4][NX], vb[4][NX];
-    load_tile(0, ka, va);
+    f32x4 va[4][NW], vb[4][NW];
+    load_k(0, ka);
+    load_v(0, va);
     for (int k = 0;; k += 2) {
-      if (k + 1 < ntiles) load_tile(k + 1, kb, vb);
+      if (k + 1 < ntiles) {
+        load_k(k + 1, kb);
+        load_v(k + 1, vb);
+      }
       compute_tile(k, ka, va);
       if (k + 1 >= ntiles) break;
-      if (k + 2 < ntiles) load_tile(k + 2, ka, va);
+      if (k + 2 < ntiles) {
+        load_k(k + 2, ka);
+        load_v(k + 2, va);
+      }
       compute_tile(k + 1, kb, vb);
       if (k + 2 >= ntiles) break;
     }
+    finish();
   }
 
-  __device__ __forceinline__ float l_total() const {
-    float l = l_run + shfl_xor_f(l_run, 16);
+  // The same with one register set (MFMA-bound callers, whose K/V come from the caches):
+  // tile k + 1's K is loaded after tile k's scores and its V after tile k's products,
+  // half a tile of MFMAs ahead of its use.
+  __device__ __forceinline__ void run_single(int first, int stride, int t_end) {
+    const int ntiles = begin(first, stride, t_end);
+    if (ntiles == 0) return;
+    f32x4 kk[NC], vv[4][NW], sacc[RT], p[RT];
+    load_k(0, kk);
+    load_v(0, vv);
+    for (int k = 0; k < ntiles; ++k) {
+      scores(kk, sacc);
+      if (k + 1 < ntiles) load_k(k + 1, kk);
+      softmax(k, sacc, p);
+      pv(vv, p);
+      if (k + 1 < ntiles) load_v(k + 1, vv);
+    }
+    finish();
+  }
+
+  // Register transposes: o[rt][x] then holds 4 consecutive dims from f32_dim0(x, g).
+  __device__ __forceinline__ void finish() {
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+      for (int w = 0; w < NW; ++w) {
+        f32x4 t[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+          for (int j = 0; j < 4; ++j) t[i][j] = o[rt][4 * w + j][i];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) o[rt][4 * w + i] = t[i];
+      }
+  }
+
+  __device__ __forceinline__ float l_total(int rt = 0) const {
+    float l = l_run[rt] + shfl_xor_f(l_run[rt], 16);
     return l + shfl_xor_f(l, 32);
   }
 };

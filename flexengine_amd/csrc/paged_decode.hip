@@ -359,10 +359,10 @@ __global__ __launch_bounds__(kThreads) void decode_plan_kernel(const DecodeArgs 
 
 template <int D, bool PAGE16, bool PLANNED = false, class E = Fp16, bool PAD = false>
 __global__ __launch_bounds__(kThreads)
-// (fp32 and head_dim 256: one wave per SIMD, the rest of the register file held
+// (head_dim 256: one wave per SIMD, the rest of the register file held
 // as AGPRs -- at two waves D = 256 spilled 168-388 bytes per lane to scratch and
 // ran 1.6-1.8x slower)
-__attribute__((amdgpu_waves_per_eu(kIsF32<E> || D > 128 ? 1 : (PAGE16 ? FE_DECODE_WAVES_PER_EU : 2),
+__attribute__((amdgpu_waves_per_eu(D > 128 ? 1 : (PAGE16 ? FE_DECODE_WAVES_PER_EU : 2),
                                    8)))
 void piece_decode_kernel(const DecodeArgs a) {
   using C = TileCfg<D>;
@@ -470,7 +470,7 @@ void piece_decode_kernel(const DecodeArgs a) {
     core.BS = a.BS;
     core.bs_log2 = a.bs_log2;
     core.tok_end = pc.tok_end;
-    core.limit = pc.tok_end;
+    core.limit[0] = pc.tok_end;
     core.scale_log2 = a.scale_log2;
     core.new_pos = -1;
     core.knew_row = nullptr;
@@ -489,15 +489,15 @@ void piece_decode_kernel(const DecodeArgs a) {
       for (int c = 0; c < F32Core<D, PAGE16, PAD>::NC; ++c) {
         f32x4 v = f32x4{0.f, 0.f, 0.f, 0.f};
         if (!PAD || 16 * c + 4 * g < DR) v = *reinterpret_cast<const f32x4*>(qrow + 16 * c + 4 * g);
-        core.qv[c] = n < G ? v : f32x4{0.f, 0.f, 0.f, 0.f};
+        core.qv[0][c] = n < G ? v : f32x4{0.f, 0.f, 0.f, 0.f};
       }
     }
     core.init_acc();
     core.run(t_first, kWaves, t_end);
-    m_run = core.m_run;
+    m_run = core.m_run[0];
     l_tot = core.l_total();
 #pragma unroll
-    for (int x = 0; x < C::NX; ++x) o[x] = core.o[x];
+    for (int x = 0; x < C::NX; ++x) o[x] = core.o[0][x];
   } else {
   f16x8 qv[C::NK];
   {
@@ -599,8 +599,9 @@ void piece_decode_kernel(const DecodeArgs a) {
   // ---- combine the four waves: every wave parks (o, m, l) in LDS (lane-major,
   // conflict-free); wave w then combines output tiles [w*XW, (w+1)*XW) of all
   // four in the register layout of the loop: lane (g, n) holds
-  // O[head n][16x + 4g + i], so the per-head scale factors are per lane.
+  // O[head n][dim0(x) + i], so the per-head scale factors are per lane.
   constexpr int XW = C::NX / kWaves;  // output tiles per wave
+  const auto dim0 = [g](int x) { return kIsF32<E> ? f32_dim0(x, g) : 16 * x + 4 * g; };
   f32x4 ox[XW];
   float M = kNegInf, den = 0.f;
   {
@@ -639,11 +640,11 @@ void piece_decode_kernel(const DecodeArgs a) {
   const int hq = h * G + (n < G ? n : G - 1);
   if (!split) {
     if (n < G) {
-      const int64_t orow = ((int64_t)b * a.Hq + hq) * DR + 4 * g;
+      const int64_t orow = ((int64_t)b * a.Hq + hq) * DR;
 #pragma unroll
       for (int xi = 0; xi < XW; ++xi)
-        if (!PAD || 16 * (w * XW + xi) + 4 * g < DR)
-          store_out4<E>(a.out, orow + 16 * (w * XW + xi), ox[xi]);
+        if (!PAD || dim0(w * XW + xi) < DR)
+          store_out4<E>(a.out, orow + dim0(w * XW + xi), ox[xi]);
     }
     FE_TL_MARK(4);  // output stores issued
     return;
@@ -653,11 +654,10 @@ void piece_decode_kernel(const DecodeArgs a) {
     if (n >= G) return;
     const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(
         a.ws_o + ((int64_t)pc.id * a.Hq + h * G) * D, 0, G * D * (int)sizeof(float), 0x00020000);
-    const uint32_t off = (uint32_t)((n * D + 4 * g) * sizeof(float));
 #pragma unroll
     for (int xi = 0; xi < XW; ++xi)
       __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, ox[xi]), r,
-                                             off + 16 * (w * XW + xi) * (uint32_t)sizeof(float),
+                                             (n * D + dim0(w * XW + xi)) * (uint32_t)sizeof(float),
                                              0, kSc1);
     if (w == 0 && g == 0) store_coherent(a.ws_lse + (int64_t)pc.id * a.Hq + hq, M + log2f(den));
   };
@@ -1404,12 +1404,18 @@ BalancedPlan plan_balanced(int batch, int hkv, int G, int block_size, int max_le
   return p;
 }
 
+// fp32 pools whose tiles are runs of one block and whose 16 rows lie within 32-bit byte
+// offsets take the tile-list form, others look up every key row
+inline bool f32_list(const DecodeArgs& a) {
+  return a.BS % kTile == 0 && (int64_t)(a.Hkv / a.hdiv) * a.dr < ((int64_t)1 << 25);
+}
+
 template <int D, class E>
 int launch_decode(const DecodeArgs& a, hipStream_t stream) {
   const dim3 grid((a.target + 2 * a.B) * a.Hkv);
   if constexpr (kIsF32<E>) {
     // fp32 pools: the fp32 engine, unplanned
-    if (a.BS % kTile == 0)
+    if (f32_list(a))
       hipLaunchKernelGGL((piece_decode_kernel<D, true, false, E>), grid, dim3(kThreads),
                          PieceLds<D>::bytes, stream, a);
     else
@@ -1436,7 +1442,7 @@ int launch_decode(const DecodeArgs& a, hipStream_t stream) {
 template <int D, class E>
 int launch_decode_padded(const DecodeArgs& a, hipStream_t stream) {
   const dim3 grid((a.target + 2 * a.B) * a.Hkv);
-  if (a.BS % kTile == 0)
+  if (kIsF32<E> ? f32_list(a) : a.BS % kTile == 0)
     hipLaunchKernelGGL((piece_decode_kernel<D, true, false, E, true>), grid, dim3(kThreads),
                        PieceLds<D>::bytes, stream, a);
   else if constexpr (kIsF32<E>)

@@ -63,6 +63,8 @@ constexpr int kMergeRows = 4;
 // below it the extra blocks of RT = 1 fill the CUs better (measured: 1377 new tokens
 // x 12 heads run slower with RT = 2).
 constexpr int kRt2Blocks = 512;
+// fp32 prefill: (token, query head) rows from which a workgroup takes two row tiles
+constexpr int64_t kF32Rt2Rows = 20480;
 
 template <int D, int RT>
 struct PCfg {
@@ -564,11 +566,17 @@ void prefill_kernel(const PrefillArgs a) {
 // ---------------------------------------------------------------------------
 //
 // The rows of a sequence's KV-head group in the tile kernel's order (row r:
-// token r / G, query head hG + r % G), 16 per wave and 64 per workgroup.  Each
-// wave walks every key tile up to its last row's position on the fp32 engine
-// (F32Core: fp32 products on v_mfma_f32_16x16x4_f32, fp32 softmax), every
-// column masking the keys past its own position, then normalises and stores
-// its 16 rows: no LDS, no key splits.
+// token r / G, query head hG + r % G), 16 * RT per workgroup.  The workgroup's
+// four waves take the row block's 16-key tiles in turn (wave w: tiles w, w + 4,
+// ...) on the fp32 engine (F32Core: fp32 products on v_mfma_f32_16x16x4_f32, fp32
+// softmax), every column masking the keys past its own position, and combine their
+// states in LDS.
+//
+// Bound by the fp32 MFMAs (64 of 32 cycles per 16 x 16 tile at D = 128).  The first form
+// gave each wave 16 rows over all their keys: a few hundred rows left most of the chip
+// idle behind the longest rows.  At 12/2 heads of 128: 584 tokens over 2090
+// cached in 3 chunks 182 -> 50 us, four chunks of 266-434 over 1208-3012 cached 386 ->
+// 202 us (47 -> 90 TFLOP/s of the 154 that a large fp32 matrix product reaches).
 //
 // CASCADE: the prefix pass of the fp32 shared-prefix decode.  "Sequence" s is
 // a group of decode rows (locate_rows' cascade mode), every row reads the
@@ -579,9 +587,23 @@ void prefill_kernel(const PrefillArgs a) {
 //
 // PAD: head_dim a.dr below D (a multiple of 8): q, the pools and the output laid
 // out by a.dr, the dims past it zeros in q, K and V and never stored.
-template <int D, bool LIST, bool CASCADE = false, bool PAD = false>
-__global__ __launch_bounds__(kThreads) void prefill_f32_kernel(const PrefillArgs a) {
-  constexpr int ROWS = kWaves * 16;
+template <int D, int RT>
+struct F32Lds {
+  static constexpr int NX = D / 16;
+  static constexpr size_t park = 0;  // [kWaves][RT * NX][64] x 16 bytes
+  static constexpr size_t park_m = park + (size_t)kWaves * RT * NX * kWave * 16;
+  static constexpr size_t park_l = park_m + (size_t)kWaves * RT * kWave * sizeof(float);
+  static constexpr size_t bytes = park_l + (size_t)kWaves * RT * kWave * sizeof(float);
+};
+
+template <int D, bool LIST, bool CASCADE, bool PAD, int RT>
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(RT == 1 ? 3 : 2, 8)))
+void prefill_f32_kernel(const PrefillArgs a) {
+  using Core = F32Core<D, LIST, PAD, RT>;
+  using Lds = F32Lds<D, RT>;
+  constexpr int ROWS = 16 * RT;
+  constexpr int NX = Core::NX;
+  extern __shared__ __align__(16) unsigned char smem[];
   const int DR = PAD ? a.dr : D;
   if constexpr (CASCADE) {
     if (blockIdx.x == gridDim.x - 1) {
@@ -589,8 +611,10 @@ __global__ __launch_bounds__(kThreads) void prefill_f32_kernel(const PrefillArgs
       return;
     }
   }
-  const int item = blockIdx.x / a.Hkv;
-  const int h = blockIdx.x - item * a.Hkv;
+  // the last row blocks of a sequence, which see the most keys, start first
+  const int items = (CASCADE ? gridDim.x - 1 : gridDim.x) / a.Hkv;
+  const int item = items - 1 - (int)blockIdx.x / a.Hkv;
+  const int h = blockIdx.x % a.Hkv;
   RowBlock rb;
   if (!locate_rows<ROWS, CASCADE>(a, item, rb)) return;
   const int G = a.G;
@@ -600,64 +624,86 @@ __global__ __launch_bounds__(kThreads) void prefill_f32_kernel(const PrefillArgs
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int total_rows = rb.n * G;
   const int cached = CASCADE ? 0 : (rb.ctx >= rb.n ? rb.ctx - rb.n : 0);
-  const int wr0 = rb.rb * ROWS + 16 * w;
-  if (wr0 >= total_rows) return;
-  const int r_last = min(wr0 + 16, total_rows) - 1;
-  const int row = wr0 + n;
-  const bool valid = row < total_rows;
-  const int rc = valid ? row : r_last;
+  const int r0 = rb.rb * ROWS;
+  const int r_last = min(r0 + ROWS, total_rows) - 1;
 
-  F32Core<D, LIST, PAD> core;
+  Core core;
   core.k_pool = reinterpret_cast<const float*>(a.k_pool);
   core.v_pool = reinterpret_cast<const float*>(a.v_pool);
   core.k_pool_w = nullptr;
   core.v_pool_w = nullptr;
   core.trow = a.tables + (int64_t)(CASCADE ? rb.q0 : rb.s) * a.W;
-  core.rs = a.Hkv * DR;
+  core.rs = (int64_t)a.Hkv * DR;
   core.hoff = h * DR;
   core.dr = DR;
   core.W = a.W;
   core.NB = a.NB;
   core.BS = a.BS;
   core.bs_log2 = a.bs_log2;
-  if constexpr (CASCADE) {
-    core.tok_end = rb.ctx;  // the group's prefix
-    core.limit = valid && member_len(a, rb.q0 + rc / G) > rb.ctx ? rb.ctx : 0;
-  } else {
-    core.tok_end = cached + r_last / G + 1;  // the wave's last row reads the most keys
-    core.limit = valid ? cached + rc / G + 1 : 0;
-  }
+  // the block's last row reads the most keys (cascade: the group's prefix)
+  core.tok_end = CASCADE ? rb.ctx : cached + r_last / G + 1;
   core.scale_log2 = a.scale_log2;
   core.knew_row = nullptr;
   core.vnew_row = nullptr;
   core.new_pos = -1;
-  {
+#pragma unroll
+  for (int rt = 0; rt < RT; ++rt) {
+    const int row = r0 + 16 * rt + n;
+    const bool valid = row < total_rows;
+    const int rc = valid ? row : r_last;
+    if constexpr (CASCADE)
+      core.limit[rt] = valid && member_len(a, rb.q0 + rc / G) > rb.ctx ? rb.ctx : 0;
+    else
+      core.limit[rt] = valid ? cached + rc / G + 1 : 0;
     const float* qrow = reinterpret_cast<const float*>(a.q) +
                         (int64_t)(rb.q0 + rc / G) * a.q_stride + (int64_t)(h * G + rc % G) * DR;
 #pragma unroll
-    for (int c = 0; c < F32Core<D, LIST, PAD>::NC; ++c) {
-      core.qv[c] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int c = 0; c < Core::NC; ++c) {
+      core.qv[rt][c] = f32x4{0.f, 0.f, 0.f, 0.f};
       if (!PAD || 16 * c + 4 * g < DR)
-        core.qv[c] = *reinterpret_cast<const f32x4*>(qrow + 16 * c + 4 * g);
+        core.qv[rt][c] = *reinterpret_cast<const f32x4*>(qrow + 16 * c + 4 * g);
     }
   }
   core.init_acc();
-  core.run(0, 1, (core.tok_end + kTile - 1) / kTile);
-  const float l = core.l_total();
-  const float inv = l > 0.f ? 1.f / l : 0.f;
-  if (valid) {
+  core.run_single(w, kWaves, (core.tok_end + kTile - 1) / kTile);
+
+  // ---- combine: every wave parks (o, m, l) of its rows lane-major; the (row tile,
+  // output tile) pairs are then dealt to the waves ----
+  f32x4* park = reinterpret_cast<f32x4*>(smem + Lds::park);
+  float* park_m = reinterpret_cast<float*>(smem + Lds::park_m);
+  float* park_l = reinterpret_cast<float*>(smem + Lds::park_l);
+#pragma unroll
+  for (int rt = 0; rt < RT; ++rt) {
+#pragma unroll
+    for (int x = 0; x < NX; ++x) park[((w * RT + rt) * NX + x) * kWave + lane] = core.o[rt][x];
+    park_m[(w * RT + rt) * kWave + lane] = core.m_run[rt];
+    park_l[(w * RT + rt) * kWave + lane] = core.l_total(rt);
+  }
+  __syncthreads();
+  for (int t = w; t < RT * NX; t += kWaves) {
+    const int rt = t / NX, x = t % NX;
+    const int row = r0 + 16 * rt + n;
+    float M = kNegInf;
+#pragma unroll
+    for (int v = 0; v < kWaves; ++v) M = fmaxf(M, park_m[(v * RT + rt) * kWave + lane]);
+    float den = 0.f;
+    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int v = 0; v < kWaves; ++v) {
+      const float mv = park_m[(v * RT + rt) * kWave + lane];
+      const float sc = mv == kNegInf ? 0.f : exp2f(mv - M);
+      den += sc * park_l[(v * RT + rt) * kWave + lane];
+      acc += sc * park[((v * RT + rt) * NX + x) * kWave + lane];
+    }
+    if (row >= total_rows) continue;
+    const float inv = den > 0.f ? 1.f / den : 0.f;
     const int64_t r = (int64_t)(rb.q0 + row / G) * a.Hq + h * G + row % G;
+    const int d0 = f32_dim0(x, g);
     if constexpr (CASCADE) {
-      float* orow = a.pre_o + r * D + 4 * g;
-#pragma unroll
-      for (int x = 0; x < F32Core<D, LIST, PAD>::NX; ++x)
-        *reinterpret_cast<f32x4*>(orow + 16 * x) = core.o[x] * inv;
-      if (g == 0) a.pre_lse[r] = l > 0.f ? core.m_run + log2f(l) : kNegInf;
+      *reinterpret_cast<f32x4*>(a.pre_o + r * D + d0) = acc * inv;
+      if (x == 0 && g == 0) a.pre_lse[r] = den > 0.f ? M + log2f(den) : kNegInf;
     } else {
-#pragma unroll
-      for (int x = 0; x < F32Core<D, LIST, PAD>::NX; ++x)
-        if (!PAD || 4 * g + 16 * x < DR)
-          store_out4<F32>(a.out, r * DR + 4 * g + 16 * x, core.o[x] * inv);
+      if (!PAD || d0 < DR) store_out4<F32>(a.out, r * DR + d0, acc * inv);
     }
   }
 }
@@ -2046,6 +2092,36 @@ void launch_prefill_dma(const PrefillArgs& a, hipStream_t stream) {
                        stream, a);
 }
 
+template <int D, bool CASCADE, bool PAD, int RT>
+void launch_prefill_f32_form(const PrefillArgs& a, int64_t blocks, hipStream_t stream) {
+  const dim3 grid((unsigned)(blocks * a.Hkv + (CASCADE ? 1 : 0)));
+  constexpr size_t lds = F32Lds<D, RT>::bytes;
+  // tile rows held per lane: blocks of 16k tokens, 16 rows within 32-bit byte offsets
+  if (a.BS % kTile == 0 && (int64_t)a.Hkv * a.dr < ((int64_t)1 << 25))
+    hipLaunchKernelGGL((prefill_f32_kernel<D, true, CASCADE, PAD, RT>), grid, dim3(kThreads),
+                       lds, stream, a);
+  else
+    hipLaunchKernelGGL((prefill_f32_kernel<D, false, CASCADE, PAD, RT>), grid, dim3(kThreads),
+                       lds, stream, a);
+}
+
+// Two row tiles a workgroup halve the K/V reads per product but also the workgroups.  One
+// vs two, measured: 16.5k rows 202 / 211 us, 24.6k 141 / 129, 60.8k 404 / 379, 7k 50 / 58,
+// 1.2k 28 / 47.  Eight waves on the row block instead of four: 201 / 206, 149 / 139,
+// 465 / 409, 54 / 56, 29 / 46.
+template <int D, bool CASCADE, bool PAD>
+int launch_prefill_f32(const PrefillArgs& a, hipStream_t stream) {
+  const int64_t rows = (int64_t)a.total_q * a.G;
+  const int rt = rows * a.Hkv >= kF32Rt2Rows ? 2 : 1;
+  const int64_t blocks = (rows + 16 * rt - 1) / (16 * rt) + a.S;
+  if (blocks * a.Hkv + 1 >= ((int64_t)1 << 31)) return FE_ERR_UNSUPPORTED;
+  if (rt == 2)
+    launch_prefill_f32_form<D, CASCADE, PAD, 2>(a, blocks, stream);
+  else
+    launch_prefill_f32_form<D, CASCADE, PAD, 1>(a, blocks, stream);
+  return FE_LAUNCH_STATUS();
+}
+
 constexpr int kMaxTickets = 65536;
 constexpr size_t kTicketBytes = kMaxTickets * sizeof(int);
 inline size_t align256(size_t x) { return (x + 255) & ~size_t(255); }
@@ -2204,7 +2280,7 @@ int prefill_impl(const void* q, void* out, const void* k_pool, const void* v_poo
   FE_CHECK_ARG(q && out && k_pool && v_pool && block_tables && q_offsets && context_lens);
   FE_CHECK_ARG(aligned16(q) && aligned16(out) && aligned16(k_pool) && aligned16(v_pool));
   if (f32) {
-    // fp32 pools: prefill_f32_kernel, 64 rows per workgroup, no workspace
+    // fp32 pools: prefill_f32_kernel, no workspace
     if (step_plan != nullptr) return FE_ERR_UNSUPPORTED;
     PrefillArgs a{};
     a.q = (const f16*)q;
@@ -2227,28 +2303,12 @@ int prefill_impl(const void* q, void* out, const void* k_pool, const void* v_poo
     a.KS = 1;
     a.dr = head_dim;
     a.scale_log2 = scale * kLog2e;
-    const int64_t blocks = ((int64_t)total_q * a.G + kWaves * 16 - 1) / (kWaves * 16) + num_seqs;
-    if (blocks * kv_heads >= ((int64_t)1 << 31)) return FE_ERR_UNSUPPORTED;
-    const dim3 grid((unsigned)(blocks * kv_heads));
     const hipStream_t s = (hipStream_t)stream;
-    const bool list = block_size % kTile == 0;  // tile rows held per lane
-    if (padded && dpad == 64 && list)
-      hipLaunchKernelGGL((prefill_f32_kernel<64, true, false, true>), grid, dim3(kThreads), 0, s, a);
-    else if (padded && dpad == 64)
-      hipLaunchKernelGGL((prefill_f32_kernel<64, false, false, true>), grid, dim3(kThreads), 0, s, a);
-    else if (padded && list)
-      hipLaunchKernelGGL((prefill_f32_kernel<128, true, false, true>), grid, dim3(kThreads), 0, s, a);
-    else if (padded)
-      hipLaunchKernelGGL((prefill_f32_kernel<128, false, false, true>), grid, dim3(kThreads), 0, s, a);
-    else if (head_dim == 64 && list)
-      hipLaunchKernelGGL((prefill_f32_kernel<64, true>), grid, dim3(kThreads), 0, s, a);
-    else if (head_dim == 64)
-      hipLaunchKernelGGL((prefill_f32_kernel<64, false>), grid, dim3(kThreads), 0, s, a);
-    else if (list)
-      hipLaunchKernelGGL((prefill_f32_kernel<128, true>), grid, dim3(kThreads), 0, s, a);
-    else
-      hipLaunchKernelGGL((prefill_f32_kernel<128, false>), grid, dim3(kThreads), 0, s, a);
-    return FE_LAUNCH_STATUS();
+    if (padded)
+      return dpad == 64 ? launch_prefill_f32<64, false, true>(a, s)
+                        : launch_prefill_f32<128, false, true>(a, s);
+    return head_dim == 64 ? launch_prefill_f32<64, false, false>(a, s)
+                          : launch_prefill_f32<128, false, false>(a, s);
   }
   const int nwg = stream_wgs();
   const bool dma = head_dim != 256 && !padded &&
@@ -2528,12 +2588,9 @@ int cascade_prefix_launch(CascadePrefix& c, hipStream_t stream) {
     c.out_o = a.pre_o;
     c.out_lse = a.pre_lse;
     c.splits = 1;
-    const dim3 grid(blocks * a.Hkv + 1);  // + the suffix-start workgroup
-    if (c.d == 64)
-      hipLaunchKernelGGL((prefill_f32_kernel<64, true, true>), grid, dim3(kThreads), 0, stream, a);
-    else
-      hipLaunchKernelGGL((prefill_f32_kernel<128, true, true>), grid, dim3(kThreads), 0, stream, a);
-    return FE_LAUNCH_STATUS();
+    a.dr = c.d;
+    return c.d == 64 ? launch_prefill_f32<64, true, false>(a, stream)
+                     : launch_prefill_f32<128, true, false>(a, stream);
   }
   c.out_o = a.pre_o;
   c.out_lse = a.pre_lse;

@@ -317,3 +317,44 @@ def test_f32_shared_prefix_with_page_write_and_long_prefix():
     close_f32(got, exp, "fp32 cascade, 20000-token prefix")
     plain = ops.paged_decode(d.q, d.k_pool, d.v_pool, d.block_tables, d.context_lens)
     close_f32(got, plain.cpu().numpy().astype(np.float64), "fp32 cascade vs plain")
+
+@pytest.mark.parametrize("hq,hkv,d", [(12, 2, 128), (14, 2, 64), (6, 2, 96)])
+@pytest.mark.parametrize("new,cached", [
+    ([1, 3, 16, 17], [0, 15, 16, 1]),       # fewer tiles than waves, row-tile edges
+    ([64], [4100]),                         # a wave's tile list refilled (64 tiles of its own)
+    ([1900], [33]),                         # two row tiles a workgroup at 12 and 14 heads
+])
+def test_f32_prefill_row_tile_forms(hq, hkv, d, new, cached):
+    """One and two row tiles a workgroup, waves without tiles, and list and per-row table
+    lookups (block 8), against the float64 oracle at the fp32 tolerance."""
+    g = torch.Generator().manual_seed(sum(new) + d)
+    for bs in (16, 8):
+        ctx = [n + c for n, c in zip(new, cached)]
+        pages = [-(-c // bs) for c in ctx]
+        nb, width = sum(pages) + 2, max(pages)
+        perm = torch.randperm(nb, generator=g).to(torch.int32)
+        tables, at = torch.zeros((len(new), width), dtype=torch.int32), 0
+        for s, p in enumerate(pages):
+            tables[s, :p] = perm[at:at + p]
+            at += p
+        k = torch.randn(nb, bs, hkv, d, generator=g)
+        v = torch.randn(nb, bs, hkv, d, generator=g)
+        q = torch.randn(sum(new), hq, d, generator=g)
+        offs = [0]
+        for n in new:
+            offs.append(offs[-1] + n)
+        dev = lambda t: t.to(DEV)
+        got = ops.prefill_paged(dev(q), dev(k), dev(v), dev(tables),
+                                torch.tensor(offs, dtype=torch.int32, device=DEV),
+                                torch.tensor(ctx, dtype=torch.int32, device=DEV), max(new)).cpu()
+        for s, (n, c) in enumerate(zip(new, ctx)):
+            kk = k[tables[s, :pages[s]].long()].flatten(0, 1)[:c].double()
+            vv = v[tables[s, :pages[s]].long()].flatten(0, 1)[:c].double()
+            rows = torch.arange(n) if n <= 64 else torch.arange(0, n, 37)
+            qq = q[offs[s] + rows].double().reshape(len(rows), hkv, hq // hkv, d)
+            sc = torch.einsum("rhgd,chd->rhgc", qq, kk) / d ** 0.5
+            sc.masked_fill_(torch.arange(c)[None, None, None] > (c - n + rows)[:, None, None, None],
+                            float("-inf"))
+            want = torch.einsum("rhgc,chd->rhgd", torch.softmax(sc, -1), vv).reshape(len(rows), hq, d)
+            err = (got[offs[s] + rows].double() - want).abs()
+            assert err.max() <= 2e-5 and err.mean() <= 2e-6, (bs, s, err.max(), err.mean())
