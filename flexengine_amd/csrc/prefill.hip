@@ -1082,6 +1082,14 @@ struct StreamPlan {
 // ceil(nb_max / (kMaxContrib - 2)) blocks, so a unit of nb_max blocks meets at
 // most kMaxContrib - 1 of them.
 constexpr int kMaxContrib = 32;
+// Key blocks of a workgroup's range at least, where the blocks would give less than
+// kShortRange a workgroup and the units hold kLongUnit on average.  All workgroups / this
+// rule, fp16: 100 tokens over 1000 cached (12/2 heads of 128) 44.7 / 30.1 us, 30 over 4000
+// 51.9 / 35.3, 200 and 100 over 300 and 1500 78.3 / 31.5, six times 64 over 500 47.5 / 31.6,
+// 16 over 4000 (32/8) 32.5 / 27.4.  Units of fewer blocks lose: 500 fresh tokens 28.8 / 34.1.
+constexpr int kMinRange = 6;
+constexpr int kShortRange = 3;
+constexpr int kLongUnit = 9;
 // Partials a split unit's merging lanes load per round trip.
 constexpr int kMergeBatch = 2;
 // Stream-K workgroups at most (a split unit's ticket is tickets[x0], x0 < nwg).
@@ -1090,21 +1098,30 @@ constexpr int kMaxStreamWgs = 1024;
 __device__ __forceinline__ StreamPlan stream_plan(const PrefillArgs& a) {
   const int lane = lane_id();
   StreamPlan p;
-  int T = 0;
+  int T = 0, units = 0;
   p.w0 = SeqWork{};
   int nb_max = 0;
   for (int base = 0; base < a.S; base += kWave) {
-    int blocks = 0, most = 0;
+    int blocks = 0, most = 0, rbs = 0;
     if (base + lane < a.S) {
       const SeqWork w = seq_work(a, base + lane);
       if (base == 0) p.w0 = w;
       blocks = w.tb * a.Hkv;
+      rbs = w.R * a.Hkv;
       if (w.R > 0) most = rb_blocks(a, w, w.R - 1);  // the last row block reads the most keys
     }
     T += wave_sum_i(blocks);
+    units += wave_sum_i(rbs);
     nb_max = max(nb_max, wave_max_i(most));
   }
-  const int min_range = max((nb_max + kMaxContrib - 3) / (kMaxContrib - 2), 1);
+  int min_range = max((nb_max + kMaxContrib - 3) / (kMaxContrib - 2), 1);
+  // Few blocks for the workgroups at hand, in long units (cached context): a range costs
+  // its blocks (~0.9 us each) plus opening units, storing partials and the merge, whose
+  // round trips grow with the contributors of a unit; its length then follows the root of
+  // the blocks per unit.
+  const int avg = units > 0 ? T / units : 1;
+  if (T < kShortRange * a.nwg_max && avg >= kLongUnit)
+    min_range = max(max(min_range, kMinRange), (int)sqrtf(2.f * (float)avg));
   int nwg = max(1, min(a.nwg_max, T / min_range));
   nwg = nwg >= 8 ? nwg & ~7 : nwg;
   p.rg = Ranges{T, nwg, T / nwg, T % nwg};
