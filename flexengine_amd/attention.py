@@ -31,7 +31,7 @@ BACKENDS = ("hip",)
 
 
 def _check_query(q: torch.Tensor, positions: torch.Tensor, cache) -> int:
-    if q.ndim != 3 or positions.ndim != 1 or len(q) != len(positions):
+    if q.ndim != 3 or positions.ndim != 1 or q.shape[0] != positions.shape[0]:
         raise ValueError("invalid query shape")
     if q.shape[1] % cache.layout.kv_heads:
         raise ValueError("Q heads must be a multiple of KV heads")
@@ -48,15 +48,18 @@ def attention_for_request(q: torch.Tensor, cache, layer: int, request_id: str, l
     table_list = cache.tables[request_id]
     if length <= 0 or length > len(table_list) * cache.layout.block_size:
         raise ValueError("requested length is invalid/unreserved")
-    table = torch.tensor([table_list], dtype=torch.int32).to(q.device, non_blocking=True)
     scale = 1.0 / math.sqrt(q.shape[-1])
-    if len(q) == 1:
-        ctx = torch.tensor([length], dtype=torch.int32).to(q.device, non_blocking=True)
+    # the table row, the length and the chunk's offsets in one copy to the device: three
+    # small ones took 30 us a call, most of it host time, where the kernel takes 9
+    n, pages = q.shape[0], len(table_list)
+    buf = torch.tensor([*table_list, length, 0, n], dtype=torch.int32).to(q.device,
+                                                                        non_blocking=True)
+    table, ctx, offs = buf.split((pages, 1, 2))
+    table = table.unsqueeze(0)
+    if n == 1:
         return ops.paged_decode(q, cache.k[layer], cache.v[layer], table, ctx, scale=scale)
-    ctx = torch.tensor([length], dtype=torch.int32).to(q.device, non_blocking=True)
-    offs = torch.tensor([0, len(q)], dtype=torch.int32).to(q.device, non_blocking=True)
-    return ops.prefill_paged(q.contiguous(), cache.k[layer], cache.v[layer], table, offs, ctx,
-                             len(q), scale=scale)
+    return ops.prefill_paged(q.contiguous(), cache.k[layer], cache.v[layer], table, offs, ctx, n,
+                             scale=scale)
 
 
 def context_lens_from_positions(positions: torch.Tensor, active_mask: torch.Tensor) -> torch.Tensor:

@@ -261,8 +261,8 @@ def hold_workspaces():
 def decode_workspace_bytes(batch: int, num_q_heads: int, head_dim: int, max_context: int,
                            target_splits: int = 0) -> int:
     """Workspace bytes for fe_paged_decode; max_context = table width * block size."""
-    return int(_lib.load().fe_paged_decode_workspace_size(batch, num_q_heads, head_dim,
-                                                          max_context, target_splits))
+    return _pure_size("fe_paged_decode_workspace_size", batch, num_q_heads, head_dim,
+                      max_context, target_splits)
 
 
 def decode_workspace(device: torch.device, nbytes: int, kind: str = "decode") -> torch.Tensor:
@@ -344,8 +344,8 @@ def paged_decode_plan(block_tables: torch.Tensor, context_lens: torch.Tensor, nu
     context_lens = _int32(context_lens, "context_lens")
     batch, width = block_tables.shape
     shape = (batch, int(kv_heads), width, int(block_size), int(num_blocks), int(target_splits))
-    need = int(_lib.load().fe_paged_decode_plan_size(batch, int(kv_heads), width * block_size,
-                                                      int(target_splits)))
+    need = _pure_size("fe_paged_decode_plan_size", batch, int(kv_heads), width * block_size,
+                      int(target_splits))
     if out is not None:
         if out.shape != shape:
             raise ValueError(f"plan buffer is for sizes {out.shape}, not {shape}")
@@ -490,8 +490,8 @@ def prefill_paged_plan(q_offsets: torch.Tensor, context_lens: torch.Tensor, tota
     num_seqs = context_lens.shape[0]
     shape = (num_seqs, int(total_q), int(num_q_heads), int(kv_heads), int(table_stride),
              int(block_size))
-    need = int(_lib.load().fe_prefill_plan_size(num_seqs, int(total_q), int(num_q_heads),
-                                                int(kv_heads)))
+    need = _pure_size("fe_prefill_plan_size", num_seqs, int(total_q), int(num_q_heads),
+                      int(kv_heads))
     if out is not None:
         if out.shape != shape:
             raise ValueError(f"plan buffer is for sizes {out.shape}, not {shape}")
