@@ -164,6 +164,36 @@ __device__ __forceinline__ f32x4 mma32(f16x8 a, f16x8 b, f32x4 c) {
   else
     return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
 }
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+// 32x32x16 MFMA (gfx950) on 16-bit operands of type E: lane l holds row l % 32 of A (and
+// column l % 32 of B), k = 8 * (l / 32) .. +7; its result register i is column l % 32 of
+// row 8 * (i / 4) + 4 * (l / 32) + i % 4
+template <class E>
+__device__ __forceinline__ f32x16 mma32x32(f16x8 a, f16x8 b, f32x16 c) {
+  if constexpr (__is_same(E, Bf16))
+    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, a),
+                                                   __builtin_bit_cast(bf16x8_t, b), c, 0, 0, 0);
+  else
+    return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
+}
+typedef f16 f16x2_t __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
+// c + the sum of 8 elements of type E
+template <class E>
+__device__ __forceinline__ float sum8(f16x8 v, float c) {
+  const f16 one = __is_same(E, Bf16) ? __builtin_bit_cast(f16, (__bf16)1.f) : (f16)1.f;
+  const f16x2_t ones = {one, one};
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const f16x2_t x = {v[2 * i], v[2 * i + 1]};
+    if constexpr (__is_same(E, Bf16))
+      c = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2_t, x),
+                                          __builtin_bit_cast(bf16x2_t, ones), c, false);
+    else
+      c = __builtin_amdgcn_fdot2(x, ones, c, false);
+  }
+  return c;
+}
 // fp32 -> the 16-bit bits of type E (round to nearest even)
 template <class E>
 __device__ __forceinline__ f16 to16(float x) {

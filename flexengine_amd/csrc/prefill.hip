@@ -763,6 +763,12 @@ __device__ __forceinline__ int swz_k(int r) { return D == 128 ? (r & 15) : ((r >
 template <int D>
 __device__ __forceinline__ int swz_v(int r) { return D == 128 ? ((r & 7) << 1) : (((r >> 1) & 3) << 1); }
 
+// V of the 32-row step (32 lanes read 4 consecutive rows x 64 bytes): 64-byte quads of
+// chunks move together, slot c ^ ((r & 3) << 2) for D = 128 and c ^ (((r >> 1) & 1) << 2)
+// for D = 64.
+template <int D>
+__device__ __forceinline__ int swz_v32(int r) { return D == 128 ? ((r & 3) << 2) : (((r >> 1) & 1) << 2); }
+
 // Row maxima of scores (finite or -inf, never NaN): IEEE maximum, which gfx950
 // computes three operands at a time (v_maximum3_f32) straight from the MFMA
 // results -- fmaxf would first canonicalise every operand, one v_max_f32
@@ -2063,6 +2069,303 @@ void prefix_dma_kernel(const PrefillArgs a) {
   if (g == 0) a.pre_lse[slot_row] = l > 0.f ? mm + log2f(l) : kNegInf;
 }
 
+// One staged 64-key block for a wave's 32 rows (the wide kernel's step) on
+// v_mfma_f32_32x32x16: lane (hf, n) = (lane / 32, lane % 32) holds row n.
+//   S^T[32 keys x 32 rows] = K.Q^T, two key tiles: lane (hf, n) gets, in register i, the
+//     score of key 8 (i / 4) + 4 hf + i % 4 of the tile, so a row's maximum and sum take
+//     one exchange between the lane halves;
+//   O^T[32 dims x 32 rows] += V^T.P^T, 16 keys s at a time: the probabilities of registers
+//     8 (s % 2) .. +7 are the B operand as they stand (k-slot (hf, j): key 16 s +
+//     8 (j / 4) + 4 hf + j % 4), and two transposing reads give the A operand the same
+//     keys of dim 32 X + n.
+// Base-2 online softmax with the lazy rescale (the causal mask only on blocks at or past
+// unmasked_blocks: key kb * 64 + j is masked past the row's pos), P as fp16 / bf16; l
+// sums, over this lane's keys, the rounded probabilities that multiply V.
+//
+// Bound by the issue of MFMAs and VALU work together: on gfx950 neither hides the other
+// fully, within a wave or between the two of a SIMD.  Eight 16x16x32 MFMAs, 32 FMAs and 8
+// exponentials took 248 ns for two waves, the same products on four 32x32x16 227 ns; the
+// 16-row form also spends 20 more VALU instructions per block on maxima and mask bounds
+// and 4 MFMAs on the row sums.
+template <int D, class E>
+__device__ __forceinline__ void dma_block32(int kb, const unsigned char* kbase,
+                                            const unsigned char* vbase, int unmasked_blocks,
+                                            float scale_log2, const f16x8 (&qv)[D / 16], int pos,
+                                            float& m_run, float& l, f32x16 (&o)[D / 32]) {
+  using P = DCfg<D>;
+  constexpr int NC = D / 16, NT = D / 32;
+  const int lane = lane_id();
+  const int hf = lane >> 5;
+  const int n = lane & 31;
+  f16x8 kf[2][NC];
+#pragma unroll
+  for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+    for (int c = 0; c < NC; ++c)
+      kf[kt][c] = *reinterpret_cast<const f16x8*>(kbase + (32 * kt + n) * P::ROWB +
+                                                  (((2 * c + hf) ^ swz_k<D>(n)) * 16));
+  f32x16 st[2];
+#pragma unroll
+  for (int kt = 0; kt < 2; ++kt) st[kt] = f32x16{};
+  // the scheduler would otherwise interleave the reads with the MFMAs to save registers,
+  // and each MFMA would wait for its read
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int c = 0; c < NC; ++c)
+#pragma unroll
+    for (int kt = 0; kt < 2; ++kt) st[kt] = mma32x32<E>(kf[kt][c], qv[c], st[kt]);
+  const int l16 = lane & 15;
+  const int vrow = 4 * hf + (l16 >> 2);
+  const int vchunk = 2 * ((lane >> 4) & 1) + ((l16 & 3) >> 1);
+  const int vswz = swz_v32<D>(vrow);
+  auto vfrag = [&](int s, int x) __attribute__((always_inline)) {
+    const unsigned char* vb = vbase + (16 * s + vrow) * P::ROWB + (l16 & 1) * 8;
+    const unsigned char* vh = vbase + (16 * s + 8 + vrow) * P::ROWB + (l16 & 1) * 8;
+    const int slot = (4 * x + vchunk) ^ vswz;
+    const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(vb + slot * 16));
+    const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(vh + slot * 16));
+    const f16x4 l4 = __builtin_bit_cast(f16x4, lo), h4 = __builtin_bit_cast(f16x4, hi);
+    return f16x8{l4[0], l4[1], l4[2], l4[3], h4[0], h4[1], h4[2], h4[3]};
+  };
+  // the first 32 keys' V fragments are read before the softmax, which hides their latency
+  f16x8 vf[2][NT];
+#pragma unroll
+  for (int s = 0; s < 2; ++s)
+#pragma unroll
+    for (int x = 0; x < NT; ++x) vf[s][x] = vfrag(s, x);
+
+  if (kb >= unmasked_blocks) {  // wave-uniform
+    int rel = pos - kb * kDmaKeys - 4 * hf;  // keys past it in this lane's numbering
+    // (defined here as far as the compiler knows: otherwise it hoists the comparisons and
+    // makes the branch 64 compares and selects on every block)
+    asm volatile("" : "+v"(rel));
+#pragma unroll
+    for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+      for (int i = 0; i < 16; ++i)
+        if (32 * kt + 8 * (i / 4) + i % 4 > rel) st[kt][i] = kNegInf;
+  }
+  float mx = vmax3(st[0][0], st[0][1], st[0][2]);
+#pragma unroll
+  for (int i = 3; i < 15; i += 2) mx = vmax3(mx, st[0][i], st[0][i + 1]);
+  float my = vmax3(st[1][0], st[1][1], st[1][2]);
+#pragma unroll
+  for (int i = 3; i < 15; i += 2) my = vmax3(my, st[1][i], st[1][i + 1]);
+  mx = vmax3(mx, st[0][15], vmax2(my, st[1][15]));
+  {
+    const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(mx), __float_as_uint(mx), false, false);
+    mx = vmax2(__uint_as_float(b[0]), __uint_as_float(b[1]));
+  }
+  mx *= scale_log2;
+  if (__ballot(mx > m_run + kRescaleSlack)) {  // wave-uniform
+    const float m_new = fmaxf(m_run, mx);
+    const float alpha = m_new == kNegInf ? 1.f : exp2_fast(m_run - m_new);
+    l *= alpha;
+#pragma unroll
+    for (int x = 0; x < NT; ++x) o[x] *= alpha;
+    m_run = m_new;
+  }
+  const float neg_m = m_run == kNegInf ? 0.f : -m_run;
+  f16x8 pb[4];
+#pragma unroll
+  for (int s = 0; s < 4; ++s) {
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+      pb[s][j] = to16<E>(exp2_fast(__builtin_fmaf(st[s / 2][8 * (s % 2) + j], scale_log2, neg_m)));
+    l = sum8<E>(pb[s], l);
+  }
+#pragma unroll
+  for (int s = 0; s < 4; ++s)
+#pragma unroll
+    for (int x = 0; x < NT; ++x) {
+      const f16x8 va = vf[s % 2][x];
+      if (s < 2) vf[s][x] = vfrag(s + 2, x);  // in flight during the next 16 keys' products
+      o[x] = mma32x32<E>(va, pb[s], o[x]);
+    }
+}
+
+// ---------------------------------------------------------------------------
+// prefill_wide_kernel: 256 rows per workgroup, for prefills of many rows
+// ---------------------------------------------------------------------------
+//
+// A long prompt under the stream-K kernel is bound by its K/V traffic and by its unit ends:
+// every 128 rows read all their keys from the L2 / Infinity Cache (4.3 GB at 8191 tokens
+// of 32/8 heads, 5.7 TB/s), and each unit costs ~14 us of opening, exchange between the
+// halves and stores.  Here the eight waves hold 32 rows each of one 256-row block and read
+// the same 64-key blocks: half the traffic, half the unit ends, no exchange.  One
+// workgroup runs one whole row block of one KV head, the longest first (later row blocks
+// see more keys), so there are no partials, tickets or workspace; the dispatcher balances
+// them over the CUs.  K and V blocks come through a four-stage LDS-DMA ring (each wave
+// brings 8 keys of every block), three blocks in flight while one is computed.
+// 8191 tokens of 32/8 heads of 128 in bf16: 758 -> 516 us (725 -> 1064 TFLOP/s of the 1352
+// that a large matrix product reaches); of 14/2 heads of 64 in fp16 299 -> 163 us.
+constexpr int kWideRows = 256;
+constexpr int kWideRun = 8;      // keys of a block each wave brings in
+
+template <int D, class E, bool PLANNED>
+__global__ __launch_bounds__(kDmaThreads) __attribute__((amdgpu_waves_per_eu(2, 2)))
+void prefill_wide_kernel(const PrefillArgs a) {
+  using P = DCfg<D>;
+  constexpr int VM_BLOCK = 2 * kWideRun / P::RPI;  // DMA instructions of one wave per block
+  static_assert(kDmaThreads / kWave * kWideRun == kDmaKeys, "the eight runs cover a block");
+  static_assert(kDmaThreads / kWave * 32 == kWideRows, "32 rows a wave");
+  // one LDS object per stage and matrix: the compiler's wait for an LDS DMA before an LDS
+  // read is then limited to reads of the object it fills
+  __shared__ __align__(16) unsigned char k0[P::MAT];
+  __shared__ __align__(16) unsigned char k1[P::MAT];
+  __shared__ __align__(16) unsigned char k2[P::MAT];
+  __shared__ __align__(16) unsigned char k3[P::MAT];
+  __shared__ __align__(16) unsigned char v0[P::MAT];
+  __shared__ __align__(16) unsigned char v1[P::MAT];
+  __shared__ __align__(16) unsigned char v2[P::MAT];
+  __shared__ __align__(16) unsigned char v3[P::MAT];
+  __shared__ int stale;  // a planned launch's verdict on the lengths
+
+  int plan_digest = 0;
+  if constexpr (PLANNED) {
+    // the plan's work split is the stream-K kernel's; its key and digest are checked here
+    // as there
+    const int* desc = a.plan + kPPlanInts;
+    const uint32_t diff_key = ((uint32_t)__builtin_amdgcn_readfirstlane(desc[0]) ^ a.plan_key_lo) |
+                              ((uint32_t)__builtin_amdgcn_readfirstlane(desc[1]) ^ a.plan_key_hi);
+    plan_digest = __builtin_amdgcn_readfirstlane(desc[kPPlanDigest]);
+    if (diff_key) {
+      refuse_plan<D, E>(a, kPPlanErrSizes);
+      return;
+    }
+  }
+  const int items = (int)gridDim.x / a.Hkv;
+  const int item = items - 1 - (int)blockIdx.x / a.Hkv;
+  const int h = (int)blockIdx.x % a.Hkv;  // (Hkv a multiple or divisor of 8: one XCD's L2 per head)
+  RowBlock rb;
+  if (!locate_rows<kWideRows, false>(a, item, rb)) {
+    if constexpr (PLANNED) {
+      if (lens_digest(a) != plan_digest) refuse_plan<D, E>(a, kPPlanErrStale);
+    }
+    return;
+  }
+  const int G = a.G;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lane = lane_id();
+  const int hf = lane >> 5;
+  const int n = lane & 31;
+  const int ctx = min(rb.ctx, a.W * a.BS);  // what the table addresses
+  const int total_rows = rb.n * G;
+  const int cached = ctx >= rb.n ? ctx - rb.n : 0;
+  const int r0 = rb.rb * kWideRows;
+  const int r_last = min(r0 + kWideRows, total_rows) - 1;
+  const int key_end = cached + r_last / G + 1;  // keys the row block reads
+  const int nb = (key_end + kDmaKeys - 1) / kDmaKeys;
+  const int wr0 = r0 + 32 * w;
+  const bool has_rows = wr0 <= r_last;
+  // blocks this wave's rows see, and those whose last key is <= every row's position
+  const int wave_nb = has_rows ? (cached + min(wr0 + 31, r_last) / G) / kDmaKeys + 1 : 0;
+  const int unmasked_blocks = (cached + min(wr0, r_last) / G + 1) / kDmaKeys;
+  const int32_t* trow = a.tables + (int64_t)rb.s * a.W;
+  // pool block of this wave's run of blocks base .. base + 63 (lane j: block base + j;
+  // pages past the table repeat its last entry, unused)
+  auto load_ids = [&](int base) __attribute__((always_inline)) {
+    int page = ((base + lane) * kDmaKeys + kWideRun * w) >> a.bs_log2;
+    page = page < a.W ? page : a.W - 1;
+    return trow[page];
+  };
+  int kb_base = 0;
+  int idv = load_ids(0);
+  const int row = wr0 + n;
+  const bool valid = row < total_rows;
+  const int rc = valid ? row : r_last;
+  const int pos = cached + rc / G;
+  f16x8 qv[D / 16];
+  {
+    const f16* qrow = a.q + (int64_t)(rb.q0 + rc / G) * a.q_stride + (h * G + rc % G) * D + 8 * hf;
+#pragma unroll
+    for (int c = 0; c < D / 16; ++c) {
+      const f16x8 v = ld16(qrow + 16 * c);
+      qv[c] = valid ? v : f16x8{};
+    }
+  }
+  const int rs = a.Hkv * D * 2;  // pool bytes from one key row to the next
+  uint32_t voff_k[P::NI], voff_v[P::NI];  // loop-invariant DMA lane offsets
+#pragma unroll
+  for (int i = 0; i < P::NI; ++i) {
+    const int rr = P::RPI * i + lane / P::CPR;
+    const int sl = lane % P::CPR;
+    voff_k[i] = (uint32_t)(rr * rs + (sl ^ swz_k<D>(kWideRun * w + rr)) * 16);
+    voff_v[i] = (uint32_t)(rr * rs + (sl ^ swz_v32<D>(kWideRun * w + rr)) * 16);
+  }
+  auto issue = [&](int kb, unsigned char* kst, unsigned char* vst) __attribute__((always_inline)) {
+    const int id = clamp_block(__builtin_amdgcn_readlane(idv, kb - kb_base), a.NB);
+    dma_run<D, kWideRun>(a, h, w, kb * kDmaKeys + kWideRun * w, key_end, id, voff_k, voff_v, kst,
+                         vst);
+  };
+  // the ids and the queries in one round trip; then the first three blocks
+  __builtin_amdgcn_s_waitcnt(kWaitVm0);
+  issue(0, k0, v0);
+  if (nb > 1) issue(1, k1, v1);
+  if (nb > 2) issue(2, k2, v2);
+  if constexpr (PLANNED) {
+    if (w == 0) {
+      const int bad = lens_digest(a) != plan_digest;
+      if (lane == 0) stale = bad;
+    }
+    __syncthreads();
+    if (stale) {  // workgroup-uniform; nothing stored yet
+      refuse_plan<D, E>(a, kPPlanErrStale);
+      return;
+    }
+  }
+
+  float m_run = kNegInf, l_run = 0.f;
+  f32x16 o[D / 32];
+#pragma unroll
+  for (int x = 0; x < D / 32; ++x) o[x] = f32x16{};
+
+  // step j: block j sits in stage j % 4; once every wave's run of it has landed and every
+  // wave is done with block j - 1, block j + 3 goes into the stage block j - 1 used
+  auto step = [&](int j, const unsigned char* kc, const unsigned char* vc, unsigned char* kn,
+                  unsigned char* vn) __attribute__((always_inline)) {
+    if (j + 2 < nb) wait_vm<2 * VM_BLOCK>();  // blocks j + 1 and j + 2 stay in flight
+    else if (j + 1 < nb) wait_vm<VM_BLOCK>();
+    else wait_vm<0>();
+    // a bare barrier: __syncthreads()'s release fence would also wait for the DMA of
+    // blocks j + 1 and j + 2.  The wait above has put this wave's run of block j in LDS;
+    // LDS operations of a wave complete in order, and the compiler fences keep every LDS
+    // access on its side of the barrier.
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    if (j + 3 < nb) {
+      if (j + 3 - kb_base >= kWave) {
+        // the next 64 blocks' ids: the wait is an s_waitcnt the compiler sees, so no path
+        // that skips this load carries a pending load into the readlane of issue()
+        kb_base = j + 3;
+        idv = load_ids(kb_base);
+        __builtin_amdgcn_s_waitcnt(kWaitVm0);
+      }
+      issue(j + 3, kn, vn);
+    }
+    if (j < wave_nb)
+      dma_block32<D, E>(j, kc, vc, unmasked_blocks, a.scale_log2, qv, pos, m_run, l_run, o);
+  };
+  for (int j = 0; j < nb; j += 4) {
+    step(j, k0, v0, k3, v3);
+    if (j + 1 < nb) step(j + 1, k1, v1, k0, v0);
+    if (j + 2 < nb) step(j + 2, k2, v2, k1, v1);
+    if (j + 3 < nb) step(j + 3, k3, v3, k2, v2);
+  }
+  const float l = l_run + shfl_xor_f(l_run, 32);
+  if (!valid) return;
+  const float inv = l > 0.f ? 1.f / l : 0.f;
+  f16* orow = a.out + ((int64_t)(rb.q0 + row / G) * a.Hq + h * G + row % G) * D + 4 * hf;
+#pragma unroll
+  for (int x = 0; x < D / 32; ++x)
+#pragma unroll
+    for (int q4 = 0; q4 < 4; ++q4) {
+      const f32x4 t = {o[x][4 * q4], o[x][4 * q4 + 1], o[x][4 * q4 + 2], o[x][4 * q4 + 3]};
+      *reinterpret_cast<f16x4*>(orow + 32 * x + 8 * q4) = to16x4<E>(t * inv);
+    }
+}
+
 inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 inline int log2_exact(int x) {
   if (x <= 0 || (x & (x - 1))) return -1;
@@ -2136,6 +2439,48 @@ int launch_prefill_f32(const PrefillArgs& a, hipStream_t stream) {
     launch_prefill_f32_form<D, CASCADE, PAD, 2>(a, blocks, stream);
   else
     launch_prefill_f32_form<D, CASCADE, PAD, 1>(a, blocks, stream);
+  return FE_LAUNCH_STATUS();
+}
+
+// Whether a prefill that the stream-K kernel takes runs on the wide kernel instead: by the
+// estimated time of each (us, D = 128), from what the host knows.  The longest context is
+// taken as what the tables address; the cached tokens as the rest of it beside the longest
+// chunk, half of that with several sequences.
+//   wide: 8 per round of workgroups and 1.7 per key block, of the longest unit or of a CU's
+//     rounds of average ones;
+//   stream-K: 24 (ranges, partials, merge), 1.02 per key block of a workgroup's range, 4.5
+//     per unit in the first range (k units with cb cached blocks: k cb + k^2 / G blocks).
+// Measured, wide / stream-K, fp16, 12/2 heads of 128: fresh prompts of 500 20.6 / 28.8,
+// 1000 32.8 / 40.5, 2048 58.5 / 58.2, 4096 109 / 148, 8191 237 / 385, eight of 500 23 / 43;
+// over cached tokens 3 x 1000 + 2000 82 / 70, 4000 + 4000 201 / 163, four of 266-434 over
+// 1208-3012 89 / 41.  32/8 heads: 2048 fresh 61 / 105, 4 x 200 + 500 26 / 30, 1000 + 4000
+// 126 / 89.  14/2 of 64: 4096 fresh 80 / 112.
+inline bool use_wide(int num_seqs, int total_q, int max_q_len, int G, int kv_heads,
+                     int64_t max_ctx, int cus) {
+  const double ctx = (double)max_ctx;
+  const double longest = max_q_len > 0 && max_q_len < total_q ? max_q_len : total_q;
+  double cached = ctx > longest ? ctx - longest : 0.;
+  if (num_seqs > 1) cached *= 0.5;
+  const double rows = (double)total_q * G;
+  const double avg = (cached + 0.5 * total_q / num_seqs) / kDmaKeys + 1.;
+  const double rounds = ceil((rows / kWideRows + 0.5 * num_seqs) * kv_heads / cus);
+  const double nb_max = ceil(ctx / kDmaKeys);
+  const double t_wide = 8. * rounds + 1.7 * fmax(nb_max, avg * rounds);
+  const double range = (rows / kDmaRows + num_seqs) * kv_heads * avg / cus;
+  const double cb = cached / kDmaKeys;
+  const double k = 0.5 * G * (sqrt(cb * cb + 4. * range / G) - cb);
+  const double t_stream = 24. + 1.02 * range + 4.5 * k;
+  return t_wide < 0.95 * t_stream;
+}
+
+template <int D, class E>
+int launch_prefill_wide(const PrefillArgs& a, hipStream_t stream) {
+  const int64_t blocks = ((int64_t)a.total_q * a.G + kWideRows - 1) / kWideRows + a.S;
+  const dim3 grid((unsigned)(blocks * a.Hkv));
+  if (a.plan != nullptr)
+    hipLaunchKernelGGL((prefill_wide_kernel<D, E, true>), grid, dim3(kDmaThreads), 0, stream, a);
+  else
+    hipLaunchKernelGGL((prefill_wide_kernel<D, E, false>), grid, dim3(kDmaThreads), 0, stream, a);
   return FE_LAUNCH_STATUS();
 }
 
@@ -2380,6 +2725,12 @@ int prefill_impl(const void* q, void* out, const void* k_pool, const void* v_poo
   a.plan = (int*)step_plan;
   if (a.plan != nullptr) set_pplan_key(a);
   hipStream_t s = (hipStream_t)stream;
+  if (dma && use_wide(num_seqs, total_q, max_q_len, num_q_heads / kv_heads, kv_heads,
+                      (int64_t)table_stride * block_size, nwg)) {
+    if (bf16)
+      return head_dim == 64 ? launch_prefill_wide<64, Bf16>(a, s) : launch_prefill_wide<128, Bf16>(a, s);
+    return head_dim == 64 ? launch_prefill_wide<64, Fp16>(a, s) : launch_prefill_wide<128, Fp16>(a, s);
+  }
   if (dma && bf16) {
     if (head_dim == 64) launch_prefill_dma<64, Bf16>(a, s); else launch_prefill_dma<128, Bf16>(a, s);
   } else if (dma) {

@@ -277,3 +277,75 @@ def test_planned_prefill_checks_its_plan_and_leaves_tickets_clean():
     exp = R.prefill_reference(q.numpy(), offs.numpy(), ctx2.numpy(), kp.numpy(), vp.numpy(),
                               tables.numpy(), bs)
     assert_attention_close(got.cpu().numpy(), exp, what="after a refused plan")
+
+
+@pytest.mark.parametrize("dtype,max_tol,mean_tol", [(torch.float16, 2e-3, 2e-4),
+                                                    (torch.bfloat16, 1.6e-2, 1.6e-3)])
+@pytest.mark.parametrize("new,cached,hq,hkv,d,bs", [
+    ([1, 2, 31], [0, 3, 0], 12, 2, 128, 16),          # fewer rows than one wave's 32
+    ([63, 64, 65, 1], [0, 0, 1, 130], 4, 4, 64, 16),  # block edges, one head a group
+    ([300], [17], 32, 8, 128, 32),                    # waves whose rows end before others'
+    ([43, 0, 44], [0, 50, 5], 12, 2, 128, 16),        # 258 rows: a second row block of two
+    ([1500, 700], [0, 40], 14, 2, 64, 64),            # several row blocks, group 7
+    ([4200], [0], 16, 2, 128, 16),                    # more than 64 key blocks: ids reloaded
+    ([260], [0], 71, 1, 64, 16),                      # a group above a wave's rows
+])
+def test_prefill_rows_of_fresh_prompts_match_float64(dtype, max_tol, mean_tol, new, cached, hq, hkv,
+                                                     d, bs):
+    """Short and fresh prefills (the wide kernel), unplanned and planned, against float64;
+    the plan changes no bit."""
+    g = torch.Generator().manual_seed(sum(new) + hq)
+    ctx = [n + c for n, c in zip(new, cached)]
+    pages = [-(-c // bs) for c in ctx]
+    nb, width = sum(pages) + 2, max(pages)
+    perm = torch.randperm(nb, generator=g).to(torch.int32)
+    tables, at = torch.zeros((len(new), width), dtype=torch.int32), 0
+    for s, p in enumerate(pages):
+        tables[s, :p] = perm[at:at + p]
+        at += p
+    k = torch.randn(nb, bs, hkv, d, generator=g).to(dtype).to(DEV)
+    v = torch.randn(nb, bs, hkv, d, generator=g).to(dtype).to(DEV)
+    q = torch.randn(sum(new), hq, d, generator=g).to(dtype).to(DEV)
+    offs = [0]
+    for n in new:
+        offs.append(offs[-1] + n)
+    o = torch.tensor(offs, dtype=torch.int32, device=DEV)
+    c = torch.tensor(ctx, dtype=torch.int32, device=DEV)
+    t = tables.to(DEV)
+    got = ops.prefill_paged(q, k, v, t, o, c, max(new))
+    plan = ops.prefill_paged_plan(o, c, sum(new), hq, hkv, width, bs)
+    assert torch.equal(ops.prefill_paged(q, k, v, t, o, c, max(new), plan=plan), got)
+    assert ops.plan_error(plan) == 0
+    for s, (n, x) in enumerate(zip(new, ctx)):
+        kk = k[tables[s, :pages[s]].long()].flatten(0, 1)[:x].double()
+        vv = v[tables[s, :pages[s]].long()].flatten(0, 1)[:x].double()
+        for h in sorted({0, hq // 2, hq - 1}):
+            kh, vh = kk[:, h * hkv // hq].t().contiguous(), vv[:, h * hkv // hq].contiguous()
+            sc = q[offs[s]:offs[s + 1], h].double().contiguous() @ kh / d ** 0.5
+            sc.masked_fill_(torch.arange(x, device=DEV)[None] >
+                            torch.arange(x - n, x, device=DEV)[:, None], float("-inf"))
+            err = (got[offs[s]:offs[s + 1], h].double() - torch.softmax(sc, -1) @ vh).abs()
+            assert n == 0 or (err.max() <= max_tol and err.mean() <= mean_tol), (s, h, err.max())
+
+
+def test_wide_prefill_refuses_a_stale_plan():
+    """The wide kernel checks a plan as the stream-K kernel does: changed lengths give NaN in
+    the whole output and the stale word, other sizes the sizes word."""
+    bs, hq, hkv, d, n = 16, 12, 2, 128, 700
+    pages = n // bs + 1
+    k = torch.randn(pages, bs, hkv, d, device=DEV).half()
+    v, q = torch.randn_like(k), torch.randn(n, hq, d, device=DEV).half()
+    t = torch.arange(pages, dtype=torch.int32, device=DEV)[None].contiguous()
+    o = torch.tensor([0, n], dtype=torch.int32, device=DEV)
+    c = torch.tensor([n], dtype=torch.int32, device=DEV)
+    plan = ops.prefill_paged_plan(o, c, n, hq, hkv, pages, bs)
+    good = ops.prefill_paged(q, k, v, t, o, c, n, plan=plan)
+    c.add_(1)
+    bad = ops.prefill_paged(q, k, v, t, o, c, n, plan=plan)
+    assert bad.isnan().all() and ops.plan_error(plan) == ops.PLAN_ERR_STALE
+    c.sub_(1)
+    plan.buffer[64:68].zero_()   # the key's low word
+    bad = ops.prefill_paged(q, k, v, t, o, c, n, plan=plan)
+    assert bad.isnan().all() and ops.plan_error(plan) == ops.PLAN_ERR_SIZES
+    plan = ops.prefill_paged_plan(o, c, n, hq, hkv, pages, bs)
+    assert torch.equal(ops.prefill_paged(q, k, v, t, o, c, n, plan=plan), good)
