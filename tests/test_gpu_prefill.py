@@ -328,6 +328,26 @@ def test_prefill_rows_of_fresh_prompts_match_float64(dtype, max_tol, mean_tol, n
             assert n == 0 or (err.max() <= max_tol and err.mean() <= mean_tol), (s, h, err.max())
 
 
+def test_wide_prefill_counts_probabilities_below_the_smallest_normal():
+    """One key far above thousands of equal ones: their probabilities (5.8e-5) are subnormal in
+    fp16 and carry a fifth of the row's sum.  An error bound: probabilities to half a step of
+    2^-24 (5.2e-4) in the numerator and the sum, the output to 2^-11."""
+    bs, hq, hkv, d, n, gap = 16, 12, 2, 128, 4096, 9.75
+    q = torch.zeros(n, hq, d)
+    q[..., 0] = d ** 0.5
+    k, v = torch.zeros(n // bs, bs, hkv, d), torch.ones(n // bs, bs, hkv, d)
+    k[0, 0, :, 0], v[0, 0] = gap, 0.0
+    q, k, v = (x.half().to(DEV) for x in (q, k, v))
+    t = torch.arange(n // bs, dtype=torch.int32, device=DEV)[None].contiguous()
+    o = torch.tensor([0, n], dtype=torch.int32, device=DEV)
+    c = torch.tensor([n], dtype=torch.int32, device=DEV)
+    got = ops.prefill_paged(q, k, v, t, o, c, n).double()
+    top = float(q[0, 0, 0].double() * k[0, 0, 0, 0].double()) / d ** 0.5
+    tail = torch.arange(n, device=DEV).double()[:, None, None] * math.exp(-top)
+    exp = tail / (1.0 + tail)
+    assert ((got - exp).abs() <= (2 * 5.2e-4 + 2.0 ** -11) * exp + 2.0 ** -25).all()
+
+
 def test_wide_prefill_refuses_a_stale_plan():
     """The wide kernel checks a plan as the stream-K kernel does: changed lengths give NaN in
     the whole output and the stale word, other sizes the sizes word."""
