@@ -183,6 +183,8 @@ class Qwen2Model:
         plan = ops.prefill_paged_plan(q_offsets, ctx, len(pos_list),
                                       self.cfg.num_attention_heads, self.cfg.num_key_value_heads,
                                       width, bs)
+        ends = torch.tensor([sum(lengths[:j + 1]) - 1 for j in range(len(lengths))],
+                            dtype=torch.long).to(dev)
         x = self.embed.index_select(0, ids)
         h, _ = ops.rmsnorm(x, self.layer_weights[0].input_norm, self.cfg.rms_norm_eps)
         for layer, lw in enumerate(self.layer_weights):
@@ -190,10 +192,11 @@ class Qwen2Model:
             ops.write_kv_ragged(k, v, cache.k[layer], cache.v[layer], tables, q_offsets, ctx)
             attn = ops.prefill_paged(q, cache.k[layer], cache.v[layer], tables, q_offsets, ctx,
                                      max_q, scale=self.scale, plan=plan)
+            if layer == self.layers - 1:
+                # past the last layer's attention only the last tokens' rows reach the logits
+                x, attn = x.index_select(0, ends), attn.index_select(0, ends)
             h = self._after_attention(x, attn, lw, self._next_norm(layer))
-        ends = torch.tensor([sum(lengths[:j + 1]) - 1 for j in range(len(lengths))],
-                            dtype=torch.long).to(dev)
-        logits = self._logits(h.index_select(0, ends))
+        logits = self._logits(h)
         return [logits[j] for j in range(len(lengths))]
 
     @torch.inference_mode()
