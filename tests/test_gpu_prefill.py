@@ -348,6 +348,31 @@ def test_wide_prefill_counts_probabilities_below_the_smallest_normal():
     assert ((got - exp).abs() <= (2 * 5.2e-4 + 2.0 ** -11) * exp + 2.0 ** -25).all()
 
 
+@pytest.mark.parametrize("d,dtype", [(128, torch.float16), (64, torch.bfloat16)])
+def test_wide_prefill_never_uses_rows_past_a_context(d, dtype):
+    """NaN in every pool row past the contexts (the last page's tail, unused pages) leaves
+    the wide kernel's result as it is, bit for bit."""
+    bs, hq, hkv, new = 16, 12, 2, [700, 75]
+    pages = [-(-n // bs) for n in new]
+    g = torch.Generator().manual_seed(d)
+    k = torch.randn(sum(pages) + 3, bs, hkv, d, generator=g).to(dtype).to(DEV)
+    v = torch.randn(sum(pages) + 3, bs, hkv, d, generator=g).to(dtype).to(DEV)
+    q = torch.randn(sum(new), hq, d, generator=g).to(dtype).to(DEV)
+    t = torch.full((2, pages[0] + 1), sum(pages) + 2, dtype=torch.int32)
+    t[0, :pages[0]] = torch.arange(pages[0])
+    t[1, :pages[1]] = pages[0] + torch.arange(pages[1])
+    t = t.to(DEV)
+    o = torch.tensor([0, new[0], sum(new)], dtype=torch.int32, device=DEV)
+    c = torch.tensor(new, dtype=torch.int32, device=DEV)
+    good = ops.prefill_paged(q, k, v, t, o, c, max(new))
+    for pool in (k, v):
+        pool[sum(pages):] = float("nan")
+        pool[pages[0] - 1, new[0] % bs:] = float("nan")
+        pool[sum(pages) - 1, new[1] % bs:] = float("nan")
+    assert torch.equal(ops.prefill_paged(q, k, v, t, o, c, max(new)), good)
+    assert good.isfinite().all()
+
+
 def test_wide_prefill_refuses_a_stale_plan():
     """The wide kernel checks a plan as the stream-K kernel does: changed lengths give NaN in
     the whole output and the stale word, other sizes the sizes word."""
