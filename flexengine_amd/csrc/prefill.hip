@@ -806,6 +806,21 @@ __device__ __forceinline__ float max8(const float (&v)[4][4]) {
   return vmax3(a, b, vmax2(v[1][2], v[1][3]));
 }
 
+// The reference m that a row's scores are taken relative to (its running maximum, which may
+// lag by the slack of the lazy rescale) also sets what rounding to 16 bits costs: the largest
+// probabilities carry the error, and the largest of a block is exactly 1 if m is the block's
+// own maximum.  A kernel that cuts a row's keys into many short parts has that for free, one
+// that walks them in one pass does not: with m from the first block alone, the error of 64
+// tokens over 500 cached against 64 bits is 10% larger (bf16 2.09e-3 -> 2.30e-3), that of a
+// fresh prompt of 1000 3%.  So the first blocks of a pass may let m follow the block's
+// maximum in either direction: follow_max, where l is the row's sum relative to m, lets the
+// sums grow to 2^kFollowGrow of the largest probability at most.
+constexpr int kFollowBlocks = 16;
+constexpr float kFollowGrow = 16.f;
+__device__ __forceinline__ float follow_max(float m, float mx, float l) {
+  return fmaxf(mx, m - fmaxf(kFollowGrow - __builtin_amdgcn_logf(l), 0.f));
+}
+
 typedef __attribute__((address_space(3))) void lds_void;
 typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
 typedef __attribute__((address_space(4))) const int32_t const_i32;
@@ -858,13 +873,14 @@ __device__ __forceinline__ void dma_run(const PrefillArgs& a, int h, int w, int 
 // O^T += V^T.P^T, and the row sums from a tile of ones (every element of
 // lsum[rt] is the row's sum of P).  A move by 32 keys keeps the chunk
 // swizzles (they depend on the key row mod 16, or mod 32 halved).
+// follow (wave-uniform): the rows' reference follows the block's maximum (follow_max).
 template <int D, int RT, class E, int NKT = 4>
 __device__ __forceinline__ void dma_block(int kb, const unsigned char* kbase,
                                           const unsigned char* vbase, int unmasked_blocks,
                                           float scale_log2, const f16x8 (&qv)[RT][DCfg<D>::NC],
                                           const int (&pos)[RT], float (&m_run)[RT],
                                           f32x4 (&lsum)[RT], f32x4 (&o)[RT][DCfg<D>::NX],
-                                          int koff = 0) {
+                                          int koff = 0, bool follow = false) {
   static_assert(NKT == 4 || NKT == 2, "a whole block or one half");
   constexpr int NPS = NKT / 2;  // 32-key PV steps
   using P = DCfg<D>;
@@ -933,8 +949,9 @@ __device__ __forceinline__ void dma_block(int kb, const unsigned char* kbase,
           if (kb * kDmaKeys + koff + 16 * kt + 4 * g + i > pos[rt]) sv[kt][i] = kNegInf;
     }
     const float mx = max_over_lane_rows(NKT == 4 ? max16(sv) : max8(sv)) * scale_log2;
-    if (__ballot(mx > m_run[rt] + kRescaleSlack)) {  // wave-uniform
-      const float m_new = fmaxf(m_run[rt], mx);
+    if (__ballot(mx > m_run[rt] + (follow ? kNegInf : kRescaleSlack))) {  // wave-uniform
+      float m_new = fmaxf(m_run[rt], mx);
+      if (follow) m_new = follow_max(m_run[rt], mx, lsum[rt][0]);
       const float alpha = m_new == kNegInf ? 1.f : exp2_fast(m_run[rt] - m_new);
       lsum[rt] *= alpha;
 #pragma unroll
@@ -1064,6 +1081,7 @@ struct StreamPos {
 // and nwg < 2^13, so g * q < T and g * r < nwg^2).
 struct Ranges {
   int T, nwg, q, r;  // T = q * nwg + r
+  int longer;        // fewer workgroups than the blocks would fill (stream_plan)
   __device__ __forceinline__ int start(int g) const { return g * q + (g * r) / nwg; }
   // the workgroup whose range holds block x (0 <= x < T): a float estimate
   // within one of the answer, then exact steps
@@ -1126,11 +1144,15 @@ __device__ __forceinline__ StreamPlan stream_plan(const PrefillArgs& a) {
   // round trips grow with the contributors of a unit; its length then follows the root of
   // the blocks per unit.
   const int avg = units > 0 ? T / units : 1;
-  if (T < kShortRange * a.nwg_max && avg >= kLongUnit)
-    min_range = max(max(min_range, kMinRange), (int)sqrtf(2.f * (float)avg));
+  int longer = 0;
+  if (T < kShortRange * a.nwg_max && avg >= kLongUnit) {
+    const int range = max(kMinRange, (int)sqrtf(2.f * (float)avg));
+    longer = range > min_range;
+    min_range = max(min_range, range);
+  }
   int nwg = max(1, min(a.nwg_max, T / min_range));
   nwg = nwg >= 8 ? nwg & ~7 : nwg;
-  p.rg = Ranges{T, nwg, T / nwg, T % nwg};
+  p.rg = Ranges{T, nwg, T / nwg, T % nwg, longer};
   return p;
 }
 
@@ -1487,9 +1509,13 @@ __device__ __forceinline__ void run_units(const PrefillArgs& a, const StreamPlan
     }
 
     // ---- one block: S^T = K.Q^T, online softmax, O^T += V^T.P^T ----
+    // (longer ranges: the half's first blocks each take their own maximum, which ranges of
+    // one or two blocks have by themselves)
+    const int follow_end = pl.rg.longer ? kb_first + 2 * kFollowBlocks : 0;
     auto compute = [&](int kb, const unsigned char* kbase,
                        const unsigned char* vbase) __attribute__((always_inline)) {
-      dma_block<D, RT, E>(kb, kbase, vbase, unmasked_blocks, a.scale_log2, qv, pos, m_run, lsum, o);
+      dma_block<D, RT, E>(kb, kbase, vbase, unmasked_blocks, a.scale_log2, qv, pos, m_run, lsum, o,
+                          0, kb < follow_end);
     };
 
     // ---- pipeline: the DMA of the half's next block (kb + 2) runs while block
@@ -1684,7 +1710,7 @@ __device__ __forceinline__ void run_units(const PrefillArgs& a, const StreamPlan
 // ranges and, per workgroup, its range and first unit -- and
 // fe_prefill_paged_planned reads it with one load instead of the scans of
 // stream_plan and stream_locate.  Layout (int32): a header of kPPlanInts
-// (nwg, T, q, r of the Ranges), a descriptor of kPPlanInts (what the plan was
+// (nwg, T, q, r, longer of the Ranges), a descriptor of kPPlanInts (what the plan was
 // computed for: the 64-bit key of the sizes and tensors, the same fields in
 // the clear -- magic, the sizes, the q_offsets and context_lens addresses --,
 // a digest of their contents, and last an error word the planned kernel
@@ -1703,7 +1729,7 @@ __global__ __launch_bounds__(kWave) void prefill_plan_kernel(const PrefillArgs a
   const int lane = lane_id();
   if (blockIdx.x == 0) {
     const int digest = lens_digest(a);
-    const int hdr[4] = {nwg, pl.rg.T, pl.rg.q, pl.rg.r};
+    const int hdr[5] = {nwg, pl.rg.T, pl.rg.q, pl.rg.r, pl.rg.longer};
     const int desc[kPPlanFields] = {(int)a.plan_key_lo, (int)a.plan_key_hi, kPPlanMagic, a.S,
                                     a.total_q, a.Hq, a.Hkv, a.W, a.BS, a.nwg_max,
                                     lo32(a.q_off), hi32(a.q_off), lo32(a.ctx), hi32(a.ctx),
@@ -1711,7 +1737,7 @@ __global__ __launch_bounds__(kWave) void prefill_plan_kernel(const PrefillArgs a
     static_assert(kPPlanDigest == kPPlanFields - 1, "the digest closes the descriptor");
     int v = 0;  // zero padding and the error word
 #pragma unroll
-    for (int i = 0; i < 4; ++i) v = lane == i ? hdr[i] : v;
+    for (int i = 0; i < 5; ++i) v = lane == i ? hdr[i] : v;
 #pragma unroll
     for (int i = 0; i < kPPlanFields; ++i) v = lane == kPPlanInts + i ? desc[i] : v;
     if (lane < 2 * kPPlanInts) plan[lane] = v;
@@ -1777,7 +1803,7 @@ void prefill_dma_kernel(const PrefillArgs a) {
     }
     plan_digest = readlane_i(v, 2 * kPPlanInts + kPPlanDigest);
     pl.rg = Ranges{readlane_i(v, 16 + 1), readlane_i(v, 16 + 0), readlane_i(v, 16 + 2),
-                   readlane_i(v, 16 + 3)};
+                   readlane_i(v, 16 + 3), readlane_i(v, 16 + 4)};
     pl.w0 = SeqWork{};
     if ((int)blockIdx.x >= pl.rg.nwg || readlane_i(v, 2) == 0) {
       if (lens_digest(a) != plan_digest) refuse_plan<D, E>(a, kPPlanErrStale);
@@ -2087,11 +2113,22 @@ void prefix_dma_kernel(const PrefillArgs a) {
 // exponentials took 248 ns for two waves, the same products on four 32x32x16 227 ns; the
 // 16-row form also spends 20 more VALU instructions per block on maxima and mask bounds
 // and 4 MFMAs on the row sums.
+//
+// The reference follows the blocks' maxima (follow_max) over all blocks of a row block of up
+// to kFollowBlocks, else over the first kWideFollow, with a slack of kWideSlack after them: a
+// rescale costs 0.2 us a block.  Error against 64 bits and time, with the first block's
+// maximum and the general slack / this rule / the stream-K kernel: fresh prompts of 500 (fp16,
+// 12/2 heads of 128) 2.51e-4 20.3 us / 2.42e-4 21.6 / 2.42e-4 28.4, of 1000 (bf16) 2.03e-3
+// 32.5 / 1.94e-3 35.4 / 1.97e-3 40.2, of 8191 (32/8) 2.09e-3 517 / 2.02e-3 522 / 2.06e-3 759.
+constexpr float kWideSlack = 2.f;
+constexpr int kWideFollow = 2;
+
 template <int D, class E>
 __device__ __forceinline__ void dma_block32(int kb, const unsigned char* kbase,
                                             const unsigned char* vbase, int unmasked_blocks,
                                             float scale_log2, const f16x8 (&qv)[D / 16], int pos,
-                                            float& m_run, float& l, f32x16 (&o)[D / 32]) {
+                                            float& m_run, float& l, f32x16 (&o)[D / 32],
+                                            bool follow) {
   using P = DCfg<D>;
   constexpr int NC = D / 16, NT = D / 32;
   const int lane = lane_id();
@@ -2157,8 +2194,12 @@ __device__ __forceinline__ void dma_block32(int kb, const unsigned char* kbase,
     mx = vmax2(__uint_as_float(b[0]), __uint_as_float(b[1]));
   }
   mx *= scale_log2;
-  if (__ballot(mx > m_run + kRescaleSlack)) {  // wave-uniform
-    const float m_new = fmaxf(m_run, mx);
+  if (__ballot(mx > m_run + (follow ? kNegInf : kWideSlack))) {  // wave-uniform
+    float m_new = fmaxf(m_run, mx);
+    if (follow) {
+      const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(l), __float_as_uint(l), false, false);
+      m_new = follow_max(m_run, mx, __uint_as_float(b[0]) + __uint_as_float(b[1]));
+    }
     const float alpha = m_new == kNegInf ? 1.f : exp2_fast(m_run - m_new);
     l *= alpha;
 #pragma unroll
@@ -2315,6 +2356,7 @@ void prefill_wide_kernel(const PrefillArgs a) {
     }
   }
 
+  const int follow_end = nb <= kFollowBlocks ? kFollowBlocks : kWideFollow;
   float m_run = kNegInf, l_run = 0.f;
   f32x16 o[D / 32];
 #pragma unroll
@@ -2345,7 +2387,8 @@ void prefill_wide_kernel(const PrefillArgs a) {
       issue(j + 3, kn, vn);
     }
     if (j < wave_nb)
-      dma_block32<D, E>(j, kc, vc, unmasked_blocks, a.scale_log2, qv, pos, m_run, l_run, o);
+      dma_block32<D, E>(j, kc, vc, unmasked_blocks, a.scale_log2, qv, pos, m_run, l_run, o,
+                        j < follow_end);
   };
   for (int j = 0; j < nb; j += 4) {
     step(j, k0, v0, k3, v3);

@@ -394,3 +394,94 @@ def test_wide_prefill_refuses_a_stale_plan():
     assert bad.isnan().all() and ops.plan_error(plan) == ops.PLAN_ERR_SIZES
     plan = ops.prefill_paged_plan(o, c, n, hq, hkv, pages, bs)
     assert torch.equal(ops.prefill_paged(q, k, v, t, o, c, n, plan=plan), good)
+
+
+def _device_case(new, cached, hq, hkv, d, bs, dtype, seed, width=None):
+    """q, pools, tables (width pages, the longest context's by default), offsets and lengths of
+    a ragged prefill on the GPU, and its offsets and lengths as lists."""
+    g = torch.Generator().manual_seed(seed)
+    ctx = [n + c for n, c in zip(new, cached)]
+    pages = [-(-c // bs) for c in ctx]
+    nb = sum(pages) + 2
+    perm = torch.randperm(nb, generator=g).to(torch.int32)
+    tables, at = torch.full((len(new), width or max(pages)), int(perm[-1]), dtype=torch.int32), 0
+    for s, p in enumerate(pages):
+        tables[s, :p] = perm[at:at + p]
+        at += p
+    k, v = (torch.randn(nb, bs, hkv, d, generator=g).to(dtype).to(DEV) for _ in range(2))
+    q = torch.randn(sum(new), hq, d, generator=g).to(dtype).to(DEV)
+    offs = [0] + np.cumsum(new).tolist()
+    return (q, k, v, tables.to(DEV), torch.tensor(offs, dtype=torch.int32, device=DEV),
+            torch.tensor(ctx, dtype=torch.int32, device=DEV), offs, ctx)
+
+
+def _heads_float64(q, k, v, t, offs, ctx, heads):
+    """(sequence, head, rows, scores [n, ctx] with the causal mask, V [ctx, D]) in float64."""
+    bs, hkv, d = k.shape[1:]
+    hq = q.shape[1]
+    for s, x in enumerate(ctx):
+        n = offs[s + 1] - offs[s]
+        if n == 0:
+            continue
+        pages = t[s, :-(-x // bs)].long()
+        causal = torch.arange(x, device=DEV)[None] > torch.arange(x - n, x, device=DEV)[:, None]
+        for h in heads:
+            kh = k[pages][:, :, h * hkv // hq].reshape(-1, d)[:x].double()
+            vh = v[pages][:, :, h * hkv // hq].reshape(-1, d)[:x].double()
+            sc = q[offs[s]:offs[s + 1], h].double() @ kh.t().contiguous() / d ** 0.5
+            yield s, h, slice(offs[s], offs[s + 1]), sc.masked_fill_(causal, float("-inf")), vh
+
+
+@pytest.mark.parametrize("dtype,new,cached,hq,hkv,d,bs", [
+    (torch.bfloat16, [500], [0], 12, 2, 128, 16),            # wide: a fresh prompt
+    (torch.bfloat16, [64] * 6, [500] * 6, 12, 2, 128, 16),   # wide: chunks over cached tokens
+    (torch.float16, [100] * 16, [100] * 16, 14, 2, 64, 32),
+    (torch.float16, [100], [1000], 12, 2, 128, 16),          # stream-K, several blocks a range
+    (torch.bfloat16, [16], [4000], 32, 8, 128, 16),
+    (torch.float16, [90, 40], [3000, 2500], 14, 2, 64, 16),
+])
+def test_prefill_rounds_probabilities_relative_to_each_blocks_own_maximum(dtype, new, cached, hq, hkv,
+                                                                        d, bs):
+    """The error against 64 bits is no larger than with the probabilities of every 64-key block
+    rounded to 16 bits relative to that block's own maximum and all else exact.  (One maximum
+    per row, the first block's, is 2.5-10% worse.)  The bound's 0.5%: fp32 scores and sums move
+    a probability across a rounding boundary now and then."""
+    q, k, v, t, o, c, offs, ctx = _device_case(new, cached, hq, hkv, d, bs, dtype, sum(new) + d)
+    got = ops.prefill_paged(q, k, v, t, o, c, max(new)).double()
+    err = emu = 0.0
+    for _, h, rows, sc, vh in _heads_float64(q, k, v, t, offs, ctx, range(hq)):
+        want = torch.softmax(sc, -1) @ vh
+        m = torch.stack([b.max(-1).values for b in sc.split(64, -1)], -1)
+        top = m.max(-1, keepdim=True).values
+        num, den = torch.zeros_like(want), torch.zeros(len(want), 1, device=DEV).double()
+        for j, b in enumerate(sc.split(64, -1)):
+            mj = m[:, j:j + 1].clamp_min(-1e30)
+            p = torch.exp(b - mj).to(dtype).double()
+            w = torch.exp(mj - top)
+            num += w * (p @ vh[64 * j:64 * (j + 1)])
+            den += w * p.sum(-1, keepdim=True)
+        err += (got[rows, h] - want).square().sum().item()
+        emu += ((num / den).to(dtype).double() - want).square().sum().item()
+    assert err ** 0.5 <= 1.005 * emu ** 0.5, (err ** 0.5, emu ** 0.5)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("new,cached", [([600], [0]), ([70], [1500])])   # wide; stream-K
+def test_prefill_follows_falling_and_rising_scores(dtype, new, cached):
+    """Block maxima that fall by 12 from block to block and then rise again: the reference of
+    the probabilities follows them down no further than the sums allow, and back up."""
+    q, k, v, t, o, c, offs, ctx = _device_case(new, cached, 12, 2, 128, 16, dtype, 5)
+    x, pages = ctx[0], t[0].long()
+    step = -12.0 * (torch.arange(x, device=DEV) // 64).float()
+    step = torch.maximum(step, step.flip(0))                       # falls, then rises
+    k[..., 0] = 0
+    flat = k[pages].flatten(0, 1)
+    flat[:x, :, 0] = (step / 8.0)[:, None].to(dtype)
+    k[pages] = flat.view(-1, *k.shape[1:])
+    q[..., 0] = 8.0 * 128 ** 0.5                                   # score += step (key)
+    got = ops.prefill_paged(q, k, v, t, o, c, max(new)).double()
+    assert got.isfinite().all()
+    unit = 2.0 ** (-11 if dtype == torch.float16 else -8)  # rounding of 16-bit values: of the
+    for _, h, rows, sc, vh in _heads_float64(q, k, v, t, offs, ctx, (0, 5, 11)):  # output, and
+        err = (got[rows, h] - torch.softmax(sc, -1) @ vh).abs().max()  # of p in o and in l
+        assert err <= 3 * unit * vh.abs().max(), (h, err)
