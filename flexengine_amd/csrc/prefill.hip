@@ -1076,6 +1076,22 @@ struct StreamPos {
   int s, h, rb, kb;
   SeqWork w;
 };
+// Key blocks of a workgroup's range at least.  A range costs its blocks (~0.9 us each) and
+// opening units; a unit's merge loads the partials of all its ranges, two per round trip, so
+// with a given number of blocks the best range grows with the root of the unit's length
+// times what one partial costs, kMergeFixed + kMergeFull * (rows / 128) in blocks.  Where the
+// blocks give less than kShortRange a workgroup, such ranges leave workgroups idle and win
+// all the same, given units of kLongUnit blocks and kUnitWork rows x blocks on average.
+// Measured, one block a workgroup / this rule, us: 100 tokens over 1000 cached (fp16, 12/2
+// heads of 128) 44.4 / 29.3, 30 over 4000 51.8 / 35.7, 200 and 100 over 300 and 1500 77.9 /
+// 32.7, 16 over 4000 (32/8) 32.4 / 26.4.  Ranges of six blocks whatever the rows lost where
+// a unit has few: 8 times 8 over 600 (14/2 of 64) 14.7 / 18.5 / 13.9 with this rule, one
+// token over 640 12.1 / 16.2, two over 4000 20.5 / 24.5 (both below kUnitWork).
+constexpr int kShortRange = 3;
+constexpr int kLongUnit = 9;
+constexpr int kUnitWork = 480;
+constexpr float kMergeFixed = 0.2f;
+constexpr float kMergeFull = 1.3f;
 // The ranges of the nwg workgroups: [start(g), start(g + 1)) with start(g) =
 // floor(g * T / nwg), in 32-bit arithmetic (fe_prefill_paged keeps T < 2^31
 // and nwg < 2^13, so g * q < T and g * r < nwg^2).
@@ -1106,14 +1122,6 @@ struct StreamPlan {
 // ceil(nb_max / (kMaxContrib - 2)) blocks, so a unit of nb_max blocks meets at
 // most kMaxContrib - 1 of them.
 constexpr int kMaxContrib = 32;
-// Key blocks of a workgroup's range at least, where the blocks would give less than
-// kShortRange a workgroup and the units hold kLongUnit on average.  All workgroups / this
-// rule, fp16: 100 tokens over 1000 cached (12/2 heads of 128) 44.7 / 30.1 us, 30 over 4000
-// 51.9 / 35.3, 200 and 100 over 300 and 1500 78.3 / 31.5, six times 64 over 500 47.5 / 31.6,
-// 16 over 4000 (32/8) 32.5 / 27.4.  Units of fewer blocks lose: 500 fresh tokens 28.8 / 34.1.
-constexpr int kMinRange = 6;
-constexpr int kShortRange = 3;
-constexpr int kLongUnit = 9;
 // Partials a split unit's merging lanes load per round trip.
 constexpr int kMergeBatch = 2;
 // Stream-K workgroups at most (a split unit's ticket is tickets[x0], x0 < nwg).
@@ -1122,33 +1130,34 @@ constexpr int kMaxStreamWgs = 1024;
 __device__ __forceinline__ StreamPlan stream_plan(const PrefillArgs& a) {
   const int lane = lane_id();
   StreamPlan p;
-  int T = 0, units = 0;
+  int T = 0, nb_max = 0;
+  int units = 0, rows = 0;  // this lane's, of its sequences and one KV head
   p.w0 = SeqWork{};
-  int nb_max = 0;
   for (int base = 0; base < a.S; base += kWave) {
-    int blocks = 0, most = 0, rbs = 0;
+    int blocks = 0, most = 0;
     if (base + lane < a.S) {
       const SeqWork w = seq_work(a, base + lane);
       if (base == 0) p.w0 = w;
       blocks = w.tb * a.Hkv;
-      rbs = w.R * a.Hkv;
+      units += w.R;
+      rows += w.n * a.G;
       if (w.R > 0) most = rb_blocks(a, w, w.R - 1);  // the last row block reads the most keys
     }
     T += wave_sum_i(blocks);
-    units += wave_sum_i(rbs);
     nb_max = max(nb_max, wave_max_i(most));
   }
   int min_range = max((nb_max + kMaxContrib - 3) / (kMaxContrib - 2), 1);
-  // Few blocks for the workgroups at hand, in long units (cached context): a range costs
-  // its blocks (~0.9 us each) plus opening units, storing partials and the merge, whose
-  // round trips grow with the contributors of a unit; its length then follows the root of
-  // the blocks per unit.
-  const int avg = units > 0 ? T / units : 1;
   int longer = 0;
-  if (T < kShortRange * a.nwg_max && avg >= kLongUnit) {
-    const int range = max(kMinRange, (int)sqrtf(2.f * (float)avg));
-    longer = range > min_range;
-    min_range = max(min_range, range);
+  if (T < kShortRange * a.nwg_max) {
+    units = wave_sum_i(units);
+    rows = wave_sum_i(rows);
+    const float u = (float)max(units, 1), avg = (float)T / (u * (float)a.Hkv);
+    if (avg >= (float)kLongUnit && avg * (float)rows >= (float)kUnitWork * u) {
+      const float cost = kMergeFixed + kMergeFull * (float)rows / (u * (float)kDmaRows);
+      const int range = (int)ceilf(sqrtf(avg * cost));
+      longer = range > min_range;
+      min_range = max(min_range, range);
+    }
   }
   int nwg = max(1, min(a.nwg_max, T / min_range));
   nwg = nwg >= 8 ? nwg & ~7 : nwg;

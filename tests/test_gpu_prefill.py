@@ -485,3 +485,54 @@ def test_prefill_follows_falling_and_rising_scores(dtype, new, cached):
     for _, h, rows, sc, vh in _heads_float64(q, k, v, t, offs, ctx, (0, 5, 11)):  # output, and
         err = (got[rows, h] - torch.softmax(sc, -1) @ vh).abs().max()  # of p in o and in l
         assert err <= 3 * unit * vh.abs().max(), (h, err)
+
+
+def _range_rule(new, cached, hq, hkv, nwg_max=256):
+    """(T, workgroups) of the stream-K split as its rule has them: ranges of at least
+    ceil(nb_max / 30) 64-key blocks, and where T blocks are fewer than three a workgroup, in
+    128-row units of at least nine blocks and 480 rows x blocks on average, of the root of
+    blocks x (0.2 + 1.3 rows / 128)."""
+    g = hq // hkv
+    blocks, units, rows, nb_max = 0, 0, 0, 0
+    for n, c in zip(new, cached):
+        rows += n * g
+        for rb in range(-(-n * g // 128)):
+            nb = (c + (min(128 * (rb + 1), n * g) - 1) // g) // 64 + 1
+            blocks, units, nb_max = blocks + nb, units + 1, max(nb_max, nb)
+    t, avg = blocks * hkv, blocks / max(units, 1)
+    r = max(1, -(-nb_max // 30))
+    if t < 3 * nwg_max and avg >= 9 and avg * rows >= 480 * units:
+        r = max(r, math.ceil(math.sqrt(avg * (0.2 + 1.3 * rows / (128 * units)))))
+    nwg = max(1, min(nwg_max, t // r))
+    return t, nwg & ~7 if nwg >= 8 else nwg
+
+
+@pytest.mark.parametrize("dtype,max_tol,mean_tol", [(torch.float16, 2e-3, 2e-4),
+                                                    (torch.bfloat16, 1.6e-2, 1.6e-3)])
+@pytest.mark.parametrize("new,cached,hq,hkv,d,bs", [
+    ([100], [1000], 12, 2, 128, 16),                 # longer ranges
+    ([30], [4000], 12, 2, 128, 16),
+    ([200, 100], [300, 1500], 12, 2, 128, 32),
+    ([16], [4001], 32, 8, 128, 16),
+    ([8] * 8, [600] * 8, 14, 2, 64, 32),             # few rows a unit, short ranges
+    ([5, 0, 9], [9000, 7, 3001], 71, 1, 64, 16),
+    ([1, 2], [640, 4000], 14, 2, 64, 16),            # too few rows: as with any length
+    ([1] * 5, [2841] * 5, 28, 4, 128, 16),
+    ([37] * 70, [700] * 70, 12, 2, 128, 16),         # more blocks than three a workgroup
+])
+def test_stream_k_ranges_follow_rows_and_blocks(dtype, max_tol, mean_tol, new, cached, hq, hkv, d, bs):
+    """The split of chunks over cached tokens is the rule's, planned and unplanned give the
+    same bits on one workspace call after call, and match float64."""
+    q, k, v, t, o, c, offs, ctx = _device_case(new, cached, hq, hkv, d, bs, dtype, sum(cached))
+    plan = ops.prefill_paged_plan(o, c, sum(new), hq, hkv, t.shape[1], bs)
+    header = plan.buffer[:16].view(torch.int32).tolist()
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    want_t, want_nwg = _range_rule(new, cached, hq, hkv, cus)
+    assert header[:4] == [want_nwg, want_t, want_t // want_nwg, want_t % want_nwg]
+    got = ops.prefill_paged(q, k, v, t, o, c, max(new))
+    for _ in range(2):
+        assert torch.equal(ops.prefill_paged(q, k, v, t, o, c, max(new), plan=plan), got)
+        assert torch.equal(ops.prefill_paged(q, k, v, t, o, c, max(new)), got)
+    for _, h, rows, sc, vh in _heads_float64(q, k, v, t, offs, ctx, sorted({0, hq // 2, hq - 1})):
+        err = (got[rows, h].double() - torch.softmax(sc, -1) @ vh).abs()
+        assert err.max() <= max_tol and err.mean() <= mean_tol, (h, err.max(), err.mean())
