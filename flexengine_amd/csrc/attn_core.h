@@ -521,12 +521,14 @@ struct F32Core {
 
   // The same with one register set (MFMA-bound callers, whose K/V come from the caches):
   // tile k + 1's K is loaded after tile k's scores and its V after tile k's products,
-  // half a tile of MFMAs ahead of its use.
-  __device__ __forceinline__ void run_single(int first, int stride, int t_end) {
-    const int ntiles = begin(first, stride, t_end);
+  // half a tile of MFMAs ahead of its use.  ntiles: begin()'s result, which the caller takes
+  // ahead of its query loads: K waits for the table entries and then not for the queries too.
+  __device__ __forceinline__ void run_single(int ntiles) {
     if (ntiles == 0) return;
     f32x4 kk[NC], vv[4][NW], sacc[RT], p[RT];
     load_k(0, kk);
+    // K before V: with the two interleaved the loop waits for all of V ahead of the scores
+    __builtin_amdgcn_sched_barrier(0);
     load_v(0, vv);
     for (int k = 0; k < ntiles; ++k) {
       scores(kk, sacc);
@@ -557,6 +559,33 @@ struct F32Core {
   __device__ __forceinline__ float l_total(int rt = 0) const {
     float l = l_run[rt] + shfl_xor_f(l_run[rt], 16);
     return l + shfl_xor_f(l, 32);
+  }
+
+  // After finish(): the four lanes of a row exchange 64-dim groups' chunks, so that o[x]
+  // holds the 4 dims from 16x + 4g and one store of the four covers 64 consecutive bytes.
+  __device__ __forceinline__ void to_row_order(f32x4 (&e)[NX]) const {
+#pragma unroll
+    for (int w = 0; w < NW; ++w)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        uint32_t a[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) a[i] = __float_as_uint(e[4 * w + i][j]);
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+          const auto s = __builtin_amdgcn_permlane32_swap(a[i], a[i + 2], false, false);
+          a[i] = s[0];
+          a[i + 2] = s[1];
+        }
+#pragma unroll
+        for (int i = 0; i < 4; i += 2) {
+          const auto s = __builtin_amdgcn_permlane16_swap(a[i], a[i + 1], false, false);
+          a[i] = s[0];
+          a[i + 1] = s[1];
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i) e[4 * w + i][j] = __uint_as_float(a[i]);
+      }
   }
 };
 

@@ -63,8 +63,14 @@ constexpr int kMergeRows = 4;
 // below it the extra blocks of RT = 1 fill the CUs better (measured: 1377 new tokens
 // x 12 heads run slower with RT = 2).
 constexpr int kRt2Blocks = 512;
-// fp32 prefill: (token, query head) rows from which a workgroup takes two row tiles
+// fp32 prefill: (token, query head) rows from which a workgroup takes two row tiles, if a
+// sequence and KV head then hold kF32Rt2Unit on average and their tables more than few keys
 constexpr int64_t kF32Rt2Rows = 20480;
+constexpr int kF32Rt2Unit = 48;
+// fp32 prefill, sequences of few keys (launch_prefill_f32): their longest context, and the
+// rows in all from which those of more than one key tile are treated as such
+constexpr int kF32FewKeys = 128;
+constexpr int64_t kF32FewRows = 16384;
 
 template <int D, int RT>
 struct PCfg {
@@ -100,6 +106,7 @@ struct PrefillArgs {
   int W, S, total_q, Hq, Hkv, G, BS, bs_log2, NB, KS;
   int nwg_max;       // stream-K kernel: workgroups of the launch
   int dr;            // padded tile kernel: the real head_dim (layout of q, pools, out)
+  int few_keys;      // fp32 prefill: the longest context of few keys (kF32FewKeys)
   float scale_log2;
   // shared-prefix (cascade) mode: "sequence" s is a group of decode rows
   // q_off[s] .. q_off[s+1]-1 sharing the first prefix_len[s] keys of row
@@ -122,7 +129,17 @@ struct RowBlock {
   int n;      // new rows (positions) of the sequence
   int q0;     // first query row of the sequence in q/out
   int ctx;    // context length (cached + new)
+  bool few;   // fp32 prefill: a sequence of few keys
 };
+
+// fp32 prefill: whether a sequence of `rows` (token, head) rows and ctx keys is one of few
+// keys, whose waves take ROWS rows each over all keys instead of sharing them.
+template <int ROWS>
+__device__ __forceinline__ bool few_keys(const PrefillArgs& a, int rows, int ctx) {
+  const int64_t max_keys = (int64_t)a.W * a.BS;  // what the table addresses
+  const int keys = ctx < max_keys ? ctx : (int)max_keys;
+  return keys <= kTile || (keys <= a.few_keys && rows > ROWS);
+}
 
 // Shared prefix of group s as the kernels use it: whole blocks only.
 __device__ __forceinline__ int group_prefix(const PrefillArgs& a, int s) {
@@ -136,40 +153,57 @@ __device__ __forceinline__ int member_len(const PrefillArgs& a, int b) {
   return L < a.W * a.BS ? L : a.W * a.BS;
 }
 
-// Maps a workgroup id onto (sequence, row block); false past the last block.
-template <int ROWS, bool CASCADE>
-__device__ __forceinline__ bool locate_rows(const PrefillArgs& a, int item, RowBlock& rb) {
+// Maps a workgroup id onto (sequence, row block); false past the last block.  FEW: a
+// sequence of few keys (few_keys) has row blocks of kWaves * ROWS rows (fp32 prefill).
+// PER passes of 64 sequences read their offsets and lengths in one round trip: with more
+// than 64 sequences a workgroup pays for every trip up to its own, one past the last
+// block for all of them.
+template <int ROWS, bool CASCADE, bool FEW, int PER>
+__device__ __forceinline__ bool locate_from(const PrefillArgs& a, int item, RowBlock& rb) {
   const int lane = lane_id();
   int carry = 0;
-  for (int base = 0; base < a.S; base += kWave) {
-    const int s = base + lane;
-    int q0 = 0, n = 0, cx = 0;
-    if (s < a.S) {
-      // rows outside [0, total_q) are dropped: every row the kernel touches
-      // (q, out, the context and table of a decode row) stays in its array
-      q0 = min(max(a.q_off[s], 0), a.total_q);
-      n = min(a.q_off[s + 1], a.total_q) - q0;
-      n = n > 0 ? n : 0;
+  for (int base = 0; base < a.S; base += PER * kWave) {
+    int q0[PER], q1[PER], cx[PER];
+#pragma unroll
+    for (int j = 0; j < PER; ++j) {
+      const int s = min(base + j * kWave + lane, a.S - 1);
+      q0[j] = a.q_off[s];
+      q1[j] = a.q_off[s + 1];
       // the context length (group prefix) loaded with the offsets: the hit
       // lane's is read below without another round trip
-      cx = CASCADE ? group_prefix(a, s) : clamp_len(a.ctx[s]);
+      cx[j] = CASCADE ? group_prefix(a, s) : clamp_len(a.ctx[s]);
     }
-    const int nb = (n * a.G + ROWS - 1) / ROWS;
-    const int incl = wave_scan_incl_i(nb) + carry;
-    const int excl = incl - nb;
-    const unsigned long long hit = __ballot(s < a.S && item >= excl && item < incl);
-    if (hit) {
-      const int src = __builtin_ctzll(hit);
-      rb.s = base + src;
-      rb.rb = item - readlane_i(excl, src);
-      rb.n = readlane_i(n, src);
-      rb.q0 = readlane_i(q0, src);
-      rb.ctx = readlane_i(cx, src);
-      return true;
+#pragma unroll
+    for (int j = 0; j < PER; ++j) {
+      // rows outside [0, total_q) are dropped: every row the kernel touches
+      // (q, out, the context and table of a decode row) stays in its array
+      q0[j] = min(max(q0[j], 0), a.total_q);
+      const int n = base + j * kWave + lane < a.S ? max(min(q1[j], a.total_q) - q0[j], 0) : 0;
+      const int rows = n * a.G;
+      const int few = FEW && few_keys<ROWS>(a, rows, cx[j]);
+      const int nb = few ? (rows + kWaves * ROWS - 1) / (kWaves * ROWS) : (rows + ROWS - 1) / ROWS;
+      const int incl = wave_scan_incl_i(nb) + carry;
+      const int excl = incl - nb;
+      const unsigned long long hit = __ballot(item >= excl && item < incl);
+      if (hit) {
+        const int src = __builtin_ctzll(hit);
+        rb.s = base + j * kWave + src;
+        rb.rb = item - readlane_i(excl, src);
+        rb.n = readlane_i(n, src);
+        rb.q0 = readlane_i(q0[j], src);
+        rb.ctx = readlane_i(cx[j], src);
+        rb.few = FEW && readlane_i(few, src);
+        return true;
+      }
+      carry = readlane_i(incl, kWave - 1);
     }
-    carry = readlane_i(incl, kWave - 1);
   }
   return false;
+}
+template <int ROWS, bool CASCADE, bool FEW = false>
+__device__ __forceinline__ bool locate_rows(const PrefillArgs& a, int item, RowBlock& rb) {
+  if (a.S > kWave) return locate_from<ROWS, CASCADE, FEW, 4>(a, item, rb);
+  return locate_from<ROWS, CASCADE, FEW, 1>(a, item, rb);
 }
 
 // Cascade mode: the decode row b shares group s's prefix when its context
@@ -585,6 +619,9 @@ void prefill_kernel(const PrefillArgs a) {
 // (row, query head): the normalised output in pre_o and its base-2 LSE in
 // pre_lse; the grid's last workgroup writes the suffix starts.
 //
+// FEW: a sequence of few keys (few_keys) has too few tiles to deal out, so its row blocks
+// are four times as large and each wave takes 16 * RT rows over all keys, without LDS.
+//
 // PAD: head_dim a.dr below D (a multiple of 8): q, the pools and the output laid
 // out by a.dr, the dims past it zeros in q, K and V and never stored.
 template <int D, int RT>
@@ -596,8 +633,8 @@ struct F32Lds {
   static constexpr size_t bytes = park_l + (size_t)kWaves * RT * kWave * sizeof(float);
 };
 
-template <int D, bool LIST, bool CASCADE, bool PAD, int RT>
-__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(RT == 1 ? 3 : 2, 8)))
+template <int D, bool LIST, bool CASCADE, bool PAD, int RT, bool FEW = false>
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(RT == 1 && (LIST || !PAD) ? 3 : 2, 8)))
 void prefill_f32_kernel(const PrefillArgs a) {
   using Core = F32Core<D, LIST, PAD, RT>;
   using Lds = F32Lds<D, RT>;
@@ -611,12 +648,13 @@ void prefill_f32_kernel(const PrefillArgs a) {
       return;
     }
   }
-  // the last row blocks of a sequence, which see the most keys, start first
-  const int items = (CASCADE ? gridDim.x - 1 : gridDim.x) / a.Hkv;
-  const int item = items - 1 - (int)blockIdx.x / a.Hkv;
   const int h = blockIdx.x % a.Hkv;
+  // the last row blocks of a sequence, which see the most keys, start first; workgroups
+  // past the last block start before the others, or after them where they are many (FEW)
+  const int items = (CASCADE ? gridDim.x - 1 : gridDim.x) / a.Hkv;
+  const int item = FEW ? (int)blockIdx.x / a.Hkv : items - 1 - (int)blockIdx.x / a.Hkv;
   RowBlock rb;
-  if (!locate_rows<ROWS, CASCADE>(a, item, rb)) return;
+  if (!locate_rows<ROWS, CASCADE, FEW>(a, item, rb)) return;
   const int G = a.G;
   const int lane = lane_id();
   const int g = lane >> 4;
@@ -624,7 +662,11 @@ void prefill_f32_kernel(const PrefillArgs a) {
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int total_rows = rb.n * G;
   const int cached = CASCADE ? 0 : (rb.ctx >= rb.n ? rb.ctx - rb.n : 0);
-  const int r0 = rb.rb * ROWS;
+  const bool few = FEW && rb.few;  // workgroup-uniform
+  const int block_rows = few ? kWaves * ROWS : ROWS;
+  const int block = FEW ? (total_rows - 1) / block_rows - rb.rb : rb.rb;
+  const int r0 = block * block_rows + (few ? w * ROWS : 0);
+  if (few && r0 >= total_rows) return;
   const int r_last = min(r0 + ROWS, total_rows) - 1;
 
   Core core;
@@ -646,6 +688,8 @@ void prefill_f32_kernel(const PrefillArgs a) {
   core.knew_row = nullptr;
   core.vnew_row = nullptr;
   core.new_pos = -1;
+  const int ntiles =
+      core.begin(few ? 0 : w, few ? 1 : kWaves, (core.tok_end + kTile - 1) / kTile);
 #pragma unroll
   for (int rt = 0; rt < RT; ++rt) {
     const int row = r0 + 16 * rt + n;
@@ -665,10 +709,28 @@ void prefill_f32_kernel(const PrefillArgs a) {
     }
   }
   core.init_acc();
-  core.run_single(w, kWaves, (core.tok_end + kTile - 1) / kTile);
+  core.run_single(ntiles);
+
+  if (few) {  // the wave's rows are complete
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt) {
+      core.to_row_order(core.o[rt]);
+      const int row = r0 + 16 * rt + n;
+      const float l = core.l_total(rt);
+      if (row >= total_rows) continue;
+      const float inv = l > 0.f ? 1.f / l : 0.f;
+      const int64_t r = (int64_t)(rb.q0 + row / G) * a.Hq + h * G + row % G;
+#pragma unroll
+      for (int x = 0; x < NX; ++x)
+        if (!PAD || 16 * x + 4 * g < DR)
+          store_out4<F32>(a.out, r * DR + 16 * x + 4 * g, core.o[rt][x] * inv);
+    }
+    return;
+  }
 
   // ---- combine: every wave parks (o, m, l) of its rows lane-major; the (row tile,
-  // output tile) pairs are then dealt to the waves ----
+  // output tile) pairs are then dealt to the waves, tile x taken as the 16 dims from 16x
+  // (lane (g, n) parked its 4 dims from f32_dim0(y, g) as tile y) ----
   f32x4* park = reinterpret_cast<f32x4*>(smem + Lds::park);
   float* park_m = reinterpret_cast<float*>(smem + Lds::park_m);
   float* park_l = reinterpret_cast<float*>(smem + Lds::park_l);
@@ -693,12 +755,12 @@ void prefill_f32_kernel(const PrefillArgs a) {
       const float mv = park_m[(v * RT + rt) * kWave + lane];
       const float sc = mv == kNegInf ? 0.f : exp2f(mv - M);
       den += sc * park_l[(v * RT + rt) * kWave + lane];
-      acc += sc * park[((v * RT + rt) * NX + x) * kWave + lane];
+      acc += sc * park[((v * RT + rt) * NX + (x & ~3) + g) * kWave + 16 * (x & 3) + n];
     }
     if (row >= total_rows) continue;
     const float inv = den > 0.f ? 1.f / den : 0.f;
     const int64_t r = (int64_t)(rb.q0 + row / G) * a.Hq + h * G + row % G;
-    const int d0 = f32_dim0(x, g);
+    const int d0 = 16 * x + 4 * g;
     if constexpr (CASCADE) {
       *reinterpret_cast<f32x4*>(a.pre_o + r * D + d0) = acc * inv;
       if (x == 0 && g == 0) a.pre_lse[r] = den > 0.f ? M + log2f(den) : kNegInf;
@@ -2464,16 +2526,16 @@ void launch_prefill_dma(const PrefillArgs& a, hipStream_t stream) {
                        stream, a);
 }
 
-template <int D, bool CASCADE, bool PAD, int RT>
+template <int D, bool CASCADE, bool PAD, int RT, bool FEW>
 void launch_prefill_f32_form(const PrefillArgs& a, int64_t blocks, hipStream_t stream) {
   const dim3 grid((unsigned)(blocks * a.Hkv + (CASCADE ? 1 : 0)));
   constexpr size_t lds = F32Lds<D, RT>::bytes;
   // tile rows held per lane: blocks of 16k tokens, 16 rows within 32-bit byte offsets
   if (a.BS % kTile == 0 && (int64_t)a.Hkv * a.dr < ((int64_t)1 << 25))
-    hipLaunchKernelGGL((prefill_f32_kernel<D, true, CASCADE, PAD, RT>), grid, dim3(kThreads),
+    hipLaunchKernelGGL((prefill_f32_kernel<D, true, CASCADE, PAD, RT, FEW>), grid, dim3(kThreads),
                        lds, stream, a);
   else
-    hipLaunchKernelGGL((prefill_f32_kernel<D, false, CASCADE, PAD, RT>), grid, dim3(kThreads),
+    hipLaunchKernelGGL((prefill_f32_kernel<D, false, CASCADE, PAD, RT, FEW>), grid, dim3(kThreads),
                        lds, stream, a);
 }
 
@@ -2481,16 +2543,47 @@ void launch_prefill_f32_form(const PrefillArgs& a, int64_t blocks, hipStream_t s
 // vs two, measured: 16.5k rows 202 / 211 us, 24.6k 141 / 129, 60.8k 404 / 379, 7k 50 / 58,
 // 1.2k 28 / 47.  Eight waves on the row block instead of four: 201 / 206, 149 / 139,
 // 465 / 409, 54 / 56, 29 / 46.
+//
+// FEW where the chunks are short on average, so that contexts of few keys are likely, and the
+// rows fill the chip in larger row blocks (one key tile is better off with them at any number).
+// Dealt tiles / larger row blocks / the one-wave-per-16-rows form before both, us: 256 fresh
+// prompts of 16 tokens (12/2 heads of 128) 32.5 / 23.1 / 27.4, 1024 of 8 95.3 / 42.1 / 82.3,
+// 64 of 64 39.0 / 28.4 / 38.6, 64 of 16 7.8 / 7.4 / 7.5; 16 of 64, below kF32FewRows, 11.5 /
+// 13.0 / 13.7; 64 of 200, above kF32FewKeys and two row tiles, 153 / 160 / 182.  The lengths
+// are known on the device only: tables wide enough for more keys cost workgroups past the
+// last row block (1024 of 8 in tables of 320 tokens 68, of 71/1 heads of 64 174 against 93).
 template <int D, bool CASCADE, bool PAD>
-int launch_prefill_f32(const PrefillArgs& a, hipStream_t stream) {
+int launch_prefill_f32(PrefillArgs a, hipStream_t stream) {
   const int64_t rows = (int64_t)a.total_q * a.G;
-  const int rt = rows * a.Hkv >= kF32Rt2Rows ? 2 : 1;
-  const int64_t blocks = (rows + 16 * rt - 1) / (16 * rt) + a.S;
+  int rt = rows * a.Hkv >= kF32Rt2Rows ? 2 : 1;
+  bool few = false;
+  if constexpr (!CASCADE) {
+    const int64_t max_keys = (int64_t)a.W * a.BS;
+    const bool fill = rows * a.Hkv >= kF32FewRows;
+    few = a.total_q <= (int64_t)kF32FewKeys * a.S && (fill || max_keys <= kTile);
+    a.few_keys = fill ? kF32FewKeys : kTile;
+    if (rows < (int64_t)kF32Rt2Unit * a.S || max_keys <= kF32FewKeys) rt = 1;
+  }
+  int64_t blocks = (rows + 16 * rt - 1) / (16 * rt) + a.S;
+  if (few && (int64_t)a.W * a.BS <= a.few_keys) {
+    // every sequence is one of few keys or holds one row block
+    const int per = kWaves * 16 * rt;
+    blocks = (rows + per - 1) / per + a.S;
+  }
   if (blocks * a.Hkv + 1 >= ((int64_t)1 << 31)) return FE_ERR_UNSUPPORTED;
+  if constexpr (!CASCADE) {
+    if (few) {
+      if (rt == 2)
+        launch_prefill_f32_form<D, CASCADE, PAD, 2, true>(a, blocks, stream);
+      else
+        launch_prefill_f32_form<D, CASCADE, PAD, 1, true>(a, blocks, stream);
+      return FE_LAUNCH_STATUS();
+    }
+  }
   if (rt == 2)
-    launch_prefill_f32_form<D, CASCADE, PAD, 2>(a, blocks, stream);
+    launch_prefill_f32_form<D, CASCADE, PAD, 2, false>(a, blocks, stream);
   else
-    launch_prefill_f32_form<D, CASCADE, PAD, 1>(a, blocks, stream);
+    launch_prefill_f32_form<D, CASCADE, PAD, 1, false>(a, blocks, stream);
   return FE_LAUNCH_STATUS();
 }
 

@@ -358,3 +358,56 @@ def test_f32_prefill_row_tile_forms(hq, hkv, d, new, cached):
             want = torch.einsum("rhgc,chd->rhgd", torch.softmax(sc, -1), vv).reshape(len(rows), hq, d)
             err = (got[offs[s] + rows].double() - want).abs()
             assert err.max() <= 2e-5 and err.mean() <= 2e-6, (bs, s, err.max(), err.mean())
+
+
+# --------------------------------------------------------------------------------------
+# chunks over few keys: a wave takes its rows over all keys (sequences of up to 128 keys and
+# more than one row tile, or of one key tile), the rest share the key tiles
+# --------------------------------------------------------------------------------------
+
+# contexts of every edge: one key tile, 128 keys, more; units within and past one row tile
+_FEW_NEW = [1, 2, 4, 5, 8, 16, 17, 31, 64, 65, 100, 120, 128]
+_FEW_CACHED = [0, 15, 12, 11, 120, 0, 111, 97, 0, 63, 28, 9, 1]
+
+
+@pytest.mark.parametrize("hq,hkv,d,bs,new,cached,wide", [
+    (32, 2, 64, 16, _FEW_NEW, _FEW_CACHED, 0),            # 17952 rows, one row tile a wave
+    (40, 2, 128, 16, _FEW_NEW, _FEW_CACHED, 0),           # 22440 rows, two
+    (32, 32, 64, 32, _FEW_NEW, _FEW_CACHED, 9),           # one head a group, wide tables
+    (36, 4, 96, 8, _FEW_NEW, _FEW_CACHED, 0),             # padded head dim, a lookup per key row
+    (40, 2, 40, 16, _FEW_NEW, _FEW_CACHED, 0),
+    (14, 2, 64, 16, [1, 7, 16, 0, 3], [0, 9, 0, 5, 13], 0),   # one key tile, few rows
+    (14, 2, 64, 16, [1, 7, 16, 0, 3], [0, 9, 0, 5, 13], 4),   # ... in wide tables
+    (12, 2, 128, 16, [6] * 290, [i % 70 for i in range(290)], 0),  # more than 256 sequences
+    (16, 2, 64, 16, [120] * 9 + [70], [8, 0, 9, 3, 8, 1, 0, 8, 7, 58], 0),  # tables of 136 keys
+    (16, 2, 64, 16, [120] * 9 + [70], [8, 0, 8, 3, 8, 1, 0, 8, 7, 58], 0),  # ... of 128
+])
+def test_f32_prefill_of_few_keys(hq, hkv, d, bs, new, cached, wide):
+    """Against float64, at the fp32 tolerance."""
+    g = torch.Generator().manual_seed(sum(new) + d)
+    ctx = [n + c for n, c in zip(new, cached)]
+    pages = [max(1, -(-c // bs)) for c in ctx]
+    nb = sum(pages) + 1
+    perm = torch.randperm(nb, generator=g).to(torch.int32)
+    tables, at = torch.full((len(new), max(pages) + wide), nb - 1, dtype=torch.int32), 0
+    for s, p in enumerate(pages):
+        tables[s, :p] = perm[at:at + p]
+        at += p
+    k, v = (torch.randn(nb, bs, hkv, d, generator=g).to(DEV) for _ in range(2))
+    q = torch.randn(sum(new), hq, d, generator=g).to(DEV)
+    offs = [0] + np.cumsum(new).tolist()
+    got = ops.prefill_paged(q, k, v, tables.to(DEV), torch.tensor(offs, dtype=torch.int32, device=DEV),
+                            torch.tensor(ctx, dtype=torch.int32, device=DEV), max(new))
+    assert got.isfinite().all()
+    for s, (n, x) in enumerate(zip(new, ctx)):
+        if n == 0 or (len(new) > 64 and s % 29 and s not in (63, 64, 255, 256, 289)):
+            continue
+        at = tables[s, :pages[s]].long()
+        qq = q[offs[s]:offs[s + 1]].double()
+        mask = torch.arange(x, device=DEV)[None] > torch.arange(x - n, x, device=DEV)[:, None]
+        for h in range(hq):
+            kh = k[at][:, :, h * hkv // hq].reshape(-1, d)[:x].double()
+            vh = v[at][:, :, h * hkv // hq].reshape(-1, d)[:x].double()
+            sc = (qq[:, h] @ kh.t().contiguous() / d ** 0.5).masked_fill_(mask, float("-inf"))
+            err = (got[offs[s]:offs[s + 1], h].double() - torch.softmax(sc, -1) @ vh).abs()
+            assert err.max() <= F32_MAX_TOL and err.mean() <= F32_MEAN_TOL, (s, h, err.max())
