@@ -197,42 +197,46 @@ __global__ void rope_qkv_kernel(Src qkv, const int64_t* __restrict__ positions,
 // 1500 rows of 12 / 2 heads of 128, 4.8 us here.
 constexpr int kRopeThreads = 128;
 constexpr int kRopeMaxHalf = 256;  // head_dim up to 512
+constexpr int kRopeManyRows = 96;
+constexpr int kRopeMaxGrid = 1 << 20;
 
 __global__ __launch_bounds__(kRopeThreads) void rope_rows_kernel(
     const f16* __restrict__ qkv, int64_t stride, const int64_t* __restrict__ positions,
     const float* __restrict__ inv_freq, f16* __restrict__ q_out, f16* __restrict__ k_out,
-    f16* __restrict__ v_out, int hq, int hkv, int d) {
+    f16* __restrict__ v_out, int rows, int hq, int hkv, int d) {
   __shared__ float cs[kRopeMaxHalf], sn[kRopeMaxHalf];
   const int half = d / 2;
-  const int row = blockIdx.x;
-  const float pos = (float)positions[row];
-  for (int i = threadIdx.x; i < half; i += kRopeThreads) {
-    const float ang = pos * inv_freq[i];
-    cs[i] = round16(cosf(ang));
-    sn[i] = round16(sinf(ang));
-  }
-  __syncthreads();
   const int chunks = half / 8;
-  const f16* src = qkv + (int64_t)row * stride;
-  for (int t = threadIdx.x; t < (hq + 2 * hkv) * chunks; t += kRopeThreads) {
-    const int hh = t / chunks;
-    const int i = (t - hh * chunks) * 8;
-    const f16x8 x1 = ld16(src + hh * d + i);
-    const f16x8 x2 = ld16(src + hh * d + half + i);
-    f16* dst = hh < hq         ? q_out + ((int64_t)row * hq + hh) * d
-               : hh < hq + hkv ? k_out + ((int64_t)row * hkv + (hh - hq)) * d
-                               : v_out + ((int64_t)row * hkv + (hh - hq - hkv)) * d;
-    f16x8 o1 = x1, o2 = x2;
-    if (hh < hq + hkv) {
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const float a = (float)x1[e], b = (float)x2[e], c = cs[i + e], s = sn[i + e];
-        o1[e] = (f16)(round16(a * c) + round16(-b * s));
-        o2[e] = (f16)(round16(b * c) + round16(a * s));
-      }
+  for (int row = blockIdx.x; row < rows; row += gridDim.x) {
+    if (row != (int)blockIdx.x) __syncthreads();  // the row before has been read
+    const float pos = (float)positions[row];
+    for (int i = threadIdx.x; i < half; i += kRopeThreads) {
+      const float ang = pos * inv_freq[i];
+      cs[i] = round16(cosf(ang));
+      sn[i] = round16(sinf(ang));
     }
-    st16(dst + i, o1);
-    st16(dst + half + i, o2);
+    __syncthreads();
+    const f16* src = qkv + (int64_t)row * stride;
+    for (int t = threadIdx.x; t < (hq + 2 * hkv) * chunks; t += kRopeThreads) {
+      const int hh = t / chunks;
+      const int i = (t - hh * chunks) * 8;
+      const f16x8 x1 = ld16(src + hh * d + i);
+      const f16x8 x2 = ld16(src + hh * d + half + i);
+      f16* dst = hh < hq         ? q_out + ((int64_t)row * hq + hh) * d
+                 : hh < hq + hkv ? k_out + ((int64_t)row * hkv + (hh - hq)) * d
+                                 : v_out + ((int64_t)row * hkv + (hh - hq - hkv)) * d;
+      f16x8 o1 = x1, o2 = x2;
+      if (hh < hq + hkv) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          const float a = (float)x1[e], b = (float)x2[e], c = cs[i + e], s = sn[i + e];
+          o1[e] = (f16)(round16(a * c) + round16(-b * s));
+          o2[e] = (f16)(round16(b * c) + round16(a * s));
+        }
+      }
+      st16(dst + i, o1);
+      st16(dst + half + i, o2);
+    }
   }
 }
 
@@ -271,6 +275,9 @@ __global__ __launch_bounds__(256) void silu_mul_rows_kernel(const f16* __restric
     st16(out + (int64_t)row * inter + e0, o);
   }
 }
+
+constexpr int kSiluMinInter = 1024;
+constexpr int64_t kSiluMinWork = 1 << 17;
 
 // 16-byte accesses at p are aligned
 inline bool al16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
@@ -332,13 +339,20 @@ extern "C" int fe_rope_qkv(const void* qkv, int64_t row_stride, int qkv_splits, 
   if (rows == 0) return FE_OK;
   FE_CHECK_ARG(qkv && positions && inv_freq && q_out && k_out && v_out);
   // rows in fp16 whose heads are whole aligned 16-byte chunks take the workgroup-per-row
-  // form; partials, other head dims and unaligned rows the element form.  Below 64 rows
-  // the chip is not filled either way and both are one short launch.
+  // form; partials, other head dims and unaligned rows the element form.  So do few rows of
+  // more chunks than a workgroup has threads, which it takes pass after pass on an idle
+  // chip.  Element / row form, us: one pass, 12/2 heads of 128, 1 row 2.50 / 2.29, 64 rows
+  // 2.73 / 2.48; several, 64/8 of 128, 1 row 2.61 / 3.72, 64 rows 3.81 / 4.02, 128 rows
+  // 5.43 / 4.18; 32/8 of 128, 64 rows 3.19 / 3.22, 128 rows 4.11 / 3.35.
+  const bool one_pass = (num_q_heads + 2 * kv_heads) * (head_dim / 16) <= kRopeThreads;
   if (qkv_splits == 0 && head_dim % 16 == 0 && head_dim / 2 <= kRopeMaxHalf && row_stride % 8 == 0 &&
-      al16(qkv) && al16(q_out) && al16(k_out) && al16(v_out)) {
-    hipLaunchKernelGGL(rope_rows_kernel, dim3(rows), dim3(kRopeThreads), 0, (hipStream_t)stream,
+      (one_pass || rows >= kRopeManyRows) && al16(qkv) && al16(q_out) && al16(k_out) &&
+      al16(v_out)) {
+    // (a launch holds fewer than 2^32 threads)
+    const int grid = rows < kRopeMaxGrid ? rows : kRopeMaxGrid;
+    hipLaunchKernelGGL(rope_rows_kernel, dim3(grid), dim3(kRopeThreads), 0, (hipStream_t)stream,
                        (const f16*)qkv, row_stride, positions, inv_freq, (f16*)q_out, (f16*)k_out,
-                       (f16*)v_out, num_q_heads, kv_heads, head_dim);
+                       (f16*)v_out, rows, num_q_heads, kv_heads, head_dim);
     return FE_LAUNCH_STATUS();
   }
   const int64_t work = (int64_t)rows * (num_q_heads + 2 * kv_heads) * (head_dim / 2);
@@ -354,9 +368,13 @@ extern "C" int fe_silu_mul(const void* gate_up, int64_t row_stride, int splits, 
   FE_CHECK_ARG(splits > 0 || row_stride >= 2 * (int64_t)inter);
   if (rows == 0) return FE_OK;
   FE_CHECK_ARG(gate_up && out);
-  // fp16 rows of whole aligned 16-byte chunks take the vector form, all others (partials,
-  // ragged widths or strides, unaligned rows) the element form
-  if (splits == 0 && inter % 8 == 0 && row_stride % 8 == 0 && al16(gate_up) && al16(out)) {
+  // fp16 rows of whole aligned 16-byte chunks take the vector form where there is work for
+  // it and the rows fill at least half of a workgroup; all others (partials, ragged widths
+  // or strides, unaligned rows) the element form.  Element / vector form, us: 16 rows of
+  // 4864 2.21 / 2.21, of 14336 2.49 / 2.24, 33 of 4864 2.35 / 2.25, 64 of 8960 3.19 / 2.68;
+  // 4 of 8960 2.17 / 2.21; 512 rows of 64 2.14 / 2.69.
+  if (splits == 0 && inter % 8 == 0 && row_stride % 8 == 0 && inter >= kSiluMinInter &&
+      (int64_t)rows * inter >= kSiluMinWork && al16(gate_up) && al16(out)) {
     const int gx = (inter / 8 + 255) / 256;
     hipLaunchKernelGGL(silu_mul_rows_kernel, dim3(gx, rows < 65535 ? rows : 65535), dim3(256), 0,
                        (hipStream_t)stream, (const f16*)gate_up, row_stride, (f16*)out, rows, inter);

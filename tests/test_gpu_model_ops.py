@@ -152,6 +152,41 @@ def test_silu_vector_and_element_forms_agree(rows, inter):
         assert torch.equal(ops.silu_mul(src).view(torch.int16), want.view(torch.int16))
 
 
+@pytest.mark.parametrize("rows,hq,hkv,d", [(95, 64, 8, 128), (96, 64, 8, 128), (97, 33, 2, 64),
+                                           (96, 1, 1, 512)])
+def test_rope_forms_agree_around_the_rule(rows, hq, hkv, d):
+    """Rows of more chunks than a workgroup has threads take the row form from 96 rows."""
+    qkv = randn(rows, (hq + 2 * hkv) * d, seed=25)
+    positions = torch.randint(0, 40000, (rows,), generator=gen(26), device=DEV)
+    inv_freq = 1.0 / 1e6 ** (torch.arange(0, d, 2, device=DEV, dtype=torch.float32) / d)
+    want = ops.rope_qkv(_off(qkv, 1), positions, inv_freq, hq, hkv, d)
+    for got, w in zip(ops.rope_qkv(qkv, positions, inv_freq, hq, hkv, d), want):
+        assert torch.equal(got, w)
+
+
+def test_rope_of_more_rows_than_a_launch_has_workgroups():
+    """2^25 + 3 rows: a workgroup a row would be 2^32 threads and more, which no launch takes."""
+    rows, d = (1 << 25) + 3, 16
+    qkv = torch.empty(rows, 3 * d, dtype=torch.float16, device=DEV).normal_(generator=gen(27))
+    positions = torch.arange(rows, device=DEV) % 40000
+    inv_freq = 1.0 / 1e6 ** (torch.arange(0, d, 2, device=DEV, dtype=torch.float32) / d)
+    got = ops.rope_qkv(qkv, positions, inv_freq, 1, 1, d)
+    edge = torch.tensor([0, 1, (1 << 20) - 1, 1 << 20, (1 << 20) + 1, 1 << 24, rows - 4, rows - 1],
+                        device=DEV)
+    want = ops.rope_qkv(_off(qkv[edge], 1), positions[edge], inv_freq, 1, 1, d)
+    for x, w in zip(got, want):
+        assert torch.equal(x[edge], w)
+
+
+@pytest.mark.parametrize("rows,inter", [(128, 1024), (127, 1024), (200, 1016), (64, 2056), (9, 20480)])
+def test_silu_forms_agree_around_the_rule(rows, inter):
+    """The vector form from 2^17 outputs in rows of 1024 and more, ragged last workgroups."""
+    gu = randn(rows, 2 * inter, seed=28, scale=3.0)
+    gu[0, 0], gu[0, 1], gu[0, inter + 2], gu[0, 3] = float("inf"), float("-inf"), float("nan"), 88.0
+    want = ops.silu_mul(_off(gu, 1))
+    assert torch.equal(ops.silu_mul(gu).view(torch.int16), want.view(torch.int16))
+
+
 @pytest.mark.parametrize("m,n,k", [(1, 2048, 1536), (3, 1536, 8960), (8, 17920, 1536),
                                    (16, 1000, 96), (17, 300, 1536), (32, 151936, 1536)])
 def test_gemm_skinny_matches_fp32_product(m, n, k):
