@@ -379,6 +379,8 @@ struct F32Core {
     const int n = lane & 15;
     const int t0 = (t_first + k * step) * kTile;
     if constexpr (LIST) {
+      // the row step is part of the lane offset: the range check that zeroes the keys past
+      // tok_end is not promised to count a scalar offset
       const __amdgpu_buffer_rsrc_t b = tile_rsrc(v_pool, k, t0);
       const uint32_t off = (uint32_t)((4 * g * (int)rs + 4 * n) * (int)sizeof(float));
 #pragma unroll
@@ -389,7 +391,7 @@ struct F32Core {
           if (!PAD || 64 * w + 4 * n < dr)
             vv[r][w] = __builtin_bit_cast(
                 f32x4, __builtin_amdgcn_raw_buffer_load_b128(
-                           b, off + 256 * w, (uint32_t)(r * (int)rs * (int)sizeof(float)), 0));
+                           b, off + (uint32_t)(r * (int)rs * (int)sizeof(float)) + 256 * w, 0, 0));
         }
     } else {
 #pragma unroll

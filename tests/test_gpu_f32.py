@@ -411,3 +411,81 @@ def test_f32_prefill_of_few_keys(hq, hkv, d, bs, new, cached, wide):
             sc = (qq[:, h] @ kh.t().contiguous() / d ** 0.5).masked_fill_(mask, float("-inf"))
             err = (got[offs[s]:offs[s + 1], h].double() - torch.softmax(sc, -1) @ vh).abs()
             assert err.max() <= F32_MAX_TOL and err.mean() <= F32_MEAN_TOL, (s, h, err.max())
+
+
+# --------------------------------------------------------------------------------------
+# pool rows past a context hold whatever was there before (PagedKVCache's pools are
+# uninitialised memory): NaN in all of them must leave every result as it is, bit for bit
+# --------------------------------------------------------------------------------------
+
+def _tail_pools(ctx, hq, hkv, d, bs, seed):
+    """Tables of len(ctx) rows, one page wider than the longest context (an unused block in
+    the entries past each row's own), clean pools, and copies whose rows past the contexts and
+    whose unused blocks hold NaN; all on the GPU."""
+    g = torch.Generator().manual_seed(seed)
+    pages = [-(-n // bs) for n in ctx]
+    nb = sum(pages) + 3
+    perm = torch.randperm(nb, generator=g).to(torch.int32)
+    tables = torch.full((len(ctx), max(pages) + 1), int(perm[-1]), dtype=torch.int32)
+    k, v = (torch.randn(nb, bs, hkv, d, generator=g) for _ in range(2))
+    kn, vn = k.clone(), v.clone()
+    at = 0
+    for s, (n, p) in enumerate(zip(ctx, pages)):
+        tables[s, :p] = perm[at:at + p]
+        at += p
+        if n % bs:
+            for pool in (kn, vn):
+                pool[int(tables[s, p - 1]), n % bs:] = float("nan")
+    for pool in (kn, vn):
+        pool[perm[at:].long()] = float("nan")
+    return [x.to(DEV) for x in (tables, k, v, kn, vn)]
+
+
+_TAIL_SHAPES = [(12, 2, 128, 16), (14, 2, 64, 32), (6, 2, 96, 16), (8, 1, 64, 8), (6, 2, 96, 8)]
+
+
+@pytest.mark.parametrize("hq,hkv,d,bs", _TAIL_SHAPES)
+def test_f32_decode_never_uses_rows_past_a_context(hq, hkv, d, bs):
+    """Every remainder of a 16-key tile, within the first tile and past many, plain and with
+    the fused page write of the last token."""
+    ctx = list(range(1, 33)) + [129 + r for r in range(16)] + [2000, 2003]
+    t, k, v, kn, vn = _tail_pools(ctx, hq, hkv, d, bs, 51 + d + bs)
+    g = torch.Generator().manual_seed(52)
+    q = torch.randn(len(ctx), hq, d, generator=g).to(DEV)
+    new = [torch.randn(len(ctx), hkv, d, generator=g).to(DEV) for _ in range(2)]
+    c = torch.tensor(ctx, dtype=torch.int32, device=DEV)
+    good, got = ops.paged_decode(q, k, v, t, c), ops.paged_decode(q, kn, vn, t, c)
+    assert good.isfinite().all() and torch.equal(got, good)
+    good = ops.paged_decode(q, k, v, t, c, k_new=new[0], v_new=new[1])
+    got = ops.paged_decode(q, kn, vn, t, c, k_new=new[0], v_new=new[1])
+    assert good.isfinite().all() and torch.equal(got, good)
+
+
+@pytest.mark.parametrize("hq,hkv,d,bs", _TAIL_SHAPES)
+def test_f32_prefill_never_uses_rows_past_a_context(hq, hkv, d, bs):
+    """Chunks whose contexts end at every remainder of a 16-key tile."""
+    new = [1, 2, 3, 4, 5, 6, 7, 9, 10, 11, 13, 14, 15, 17, 18, 35]
+    ctx = [n + c for n, c in zip(new, [0, 0, 0, 0, 0, 0, 0, 0, 40, 40, 0, 0, 0, 100, 0, 300])]
+    t, k, v, kn, vn = _tail_pools(ctx, hq, hkv, d, bs, 53 + d + bs)
+    q = torch.randn(sum(new), hq, d, generator=torch.Generator().manual_seed(54)).to(DEV)
+    o = torch.tensor([0] + np.cumsum(new).tolist(), dtype=torch.int32, device=DEV)
+    c = torch.tensor(ctx, dtype=torch.int32, device=DEV)
+    good = ops.prefill_paged(q, k, v, t, o, c, max(new))
+    got = ops.prefill_paged(q, kn, vn, t, o, c, max(new))
+    assert good.isfinite().all() and torch.equal(got, good)
+
+
+@pytest.mark.parametrize("hq,hkv,d,bs", _TAIL_SHAPES[:3])
+def test_f32_shared_prefix_never_uses_rows_past_a_context(hq, hkv, d, bs):
+    """Members ending at every remainder of a tile past a two-page prefix."""
+    members = 16
+    ctx = [2 * bs + 1 + r for r in range(members)]
+    t, k, v, kn, vn = _tail_pools(ctx, hq, hkv, d, bs, 55 + d)
+    t[:, :2] = t[0, :2]
+    q = torch.randn(members, hq, d, generator=torch.Generator().manual_seed(56)).to(DEV)
+    c = torch.tensor(ctx, dtype=torch.int32, device=DEV)
+    go = torch.tensor([0, members], dtype=torch.int32, device=DEV)
+    pl = torch.tensor([2 * bs], dtype=torch.int32, device=DEV)
+    good = ops.paged_decode_shared_prefix(q, k, v, t, c, go, pl)
+    got = ops.paged_decode_shared_prefix(q, kn, vn, t, c, go, pl)
+    assert good.isfinite().all() and torch.equal(got, good)
