@@ -65,6 +65,7 @@ SIGNATURES: dict[str, tuple] = {
 }
 SIGNATURES["fe_prefill_plan_size"] = (_sz, [_i, _i, _i, _i])
 SIGNATURES["fe_prefill_plan"] = (_i, [_p, _p, _i, _i, _i, _i, _i, _i, _p, _sz, _p])
+SIGNATURES["fe_prefill_form"] = (_i, [_i] * 10)
 SIGNATURES["fe_prefill_paged_planned"] = (
     _i, SIGNATURES["fe_prefill_paged"][1][:-1] + [_p, _sz, _p])
 # the bf16 forms take the fp16 entry points' arguments

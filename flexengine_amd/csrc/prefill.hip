@@ -2589,8 +2589,9 @@ int launch_prefill_f32(PrefillArgs a, hipStream_t stream) {
 
 // Whether a prefill that the stream-K kernel takes runs on the wide kernel instead: by the
 // estimated time of each (us, D = 128), from what the host knows.  The longest context is
-// taken as what the tables address; the cached tokens as the rest of it beside the longest
-// chunk, half of that with several sequences.
+// taken as what the tables address, so callers that know it pass tables of that width; the
+// cached tokens as the rest of it beside the longest chunk, half of that with several
+// sequences.
 //   wide: 8 per round of workgroups and 1.7 per key block, of the longest unit or of a CU's
 //     rounds of average ones;
 //   stream-K: 24 (ranges, partials, merge), 1.02 per key block of a workgroup's range, 4.5
@@ -2683,6 +2684,28 @@ inline bool stream_ok(int block_size, int table_stride, int total_q, int G, int 
          units * kv_heads * ((max_ctx + total_q) / kDmaKeys + 2) < ((int64_t)1 << 31);
 }
 
+// The kernel that takes a prefill of these sizes (FE_PREFILL_*; num_seqs and total_q > 0).
+inline int prefill_form(int num_seqs, int total_q, int max_q_len, int num_q_heads, int kv_heads,
+                        int head_dim, int block_size, int table_stride, bool f32, bool planned) {
+  // head_dim 256 in 16 bits runs on the tile kernel (one row tile per wave, no
+  // plan); other head dims on the generic kernel
+  const bool mfma256 = head_dim == 256 && !f32 && !planned;
+  // other multiples of 8 below 256 in 16 bits (no plan): the tile kernel at the
+  // next of 64 / 128 / 256, the dims past head_dim zeros
+  // (fp32: the fp32 engine at 64 / 128)
+  const int dpad = mfma_padded_head_dim(head_dim);
+  const bool padded = dpad != head_dim && !planned && (!f32 || dpad <= 128);
+  if (head_dim != 64 && head_dim != 128 && !mfma256 && !padded) return FE_PREFILL_GENERIC;
+  if (f32) return FE_PREFILL_F32;
+  const int G = num_q_heads / kv_heads, nwg = stream_wgs();
+  if (head_dim == 256 || padded ||
+      !stream_ok(block_size, table_stride, total_q, G, num_seqs, kv_heads, nwg))
+    return FE_PREFILL_TILE;
+  return use_wide(num_seqs, total_q, max_q_len, G, kv_heads, (int64_t)table_stride * block_size, nwg)
+             ? FE_PREFILL_WIDE
+             : FE_PREFILL_STREAM;
+}
+
 // Partial slots of the stream-K kernel: two per workgroup, 128 rows each.
 inline size_t stream_ws_bytes(int head_dim) {
   const size_t rows = (size_t)2 * stream_wgs() * kDmaRows;
@@ -2765,15 +2788,13 @@ int prefill_impl(const void* q, void* out, const void* k_pool, const void* v_poo
   FE_CHECK_ARG(num_seqs >= 0 && total_q >= 0 && max_q_len >= 0 && num_q_heads > 0 &&
                kv_heads > 0 && num_blocks > 0 && table_stride > 0);
   FE_CHECK_ARG(num_q_heads % kv_heads == 0);
-  // head_dim 256 in 16 bits runs on the tile kernel (one row tile per wave, no
-  // plan); other head dims on the generic kernel
-  const bool mfma256 = head_dim == 256 && !f32 && step_plan == nullptr;
-  // other multiples of 8 below 256 in 16 bits (no plan): the tile kernel at the
-  // next of 64 / 128 / 256, the dims past head_dim zeros
-  // (fp32: the fp32 engine at 64 / 128)
+  // (no sequences or no rows: use_wide's averages need one of each, and nothing is launched)
+  const int form = prefill_form(num_seqs > 0 ? num_seqs : 1, total_q > 0 ? total_q : 1, max_q_len,
+                                num_q_heads, kv_heads, head_dim, block_size, table_stride, f32,
+                                step_plan != nullptr);
   const int dpad = mfma_padded_head_dim(head_dim);
-  const bool padded = dpad != head_dim && step_plan == nullptr && (!f32 || dpad <= 128);
-  if (head_dim != 64 && head_dim != 128 && !mfma256 && !padded)
+  const bool padded = dpad != head_dim;
+  if (form == FE_PREFILL_GENERIC)
     return prefill_generic(q, out, k_pool, v_pool, num_blocks, block_tables, table_stride,
                            q_offsets, context_lens, num_seqs, total_q, num_q_heads, kv_heads,
                            head_dim, block_size, scale, (hipStream_t)stream,
@@ -2818,9 +2839,7 @@ int prefill_impl(const void* q, void* out, const void* k_pool, const void* v_poo
                           : launch_prefill_f32<128, false, false>(a, s);
   }
   const int nwg = stream_wgs();
-  const bool dma = head_dim != 256 && !padded &&
-                   stream_ok(block_size, table_stride, total_q, num_q_heads / kv_heads, num_seqs,
-                             kv_heads, nwg);
+  const bool dma = form != FE_PREFILL_TILE;  // the stream-K or the wide kernel
   // (the workspace size takes the two-tile plan: its key splits are never fewer)
   const Plan p = plan(num_seqs, total_q, num_q_heads, kv_heads, dpad != 256);
   // split-K tickets of prefill_kernel: one per (row block, KV head)
@@ -2870,8 +2889,7 @@ int prefill_impl(const void* q, void* out, const void* k_pool, const void* v_poo
   a.plan = (int*)step_plan;
   if (a.plan != nullptr) set_pplan_key(a);
   hipStream_t s = (hipStream_t)stream;
-  if (dma && use_wide(num_seqs, total_q, max_q_len, num_q_heads / kv_heads, kv_heads,
-                      (int64_t)table_stride * block_size, nwg)) {
+  if (form == FE_PREFILL_WIDE) {
     if (bf16)
       return head_dim == 64 ? launch_prefill_wide<64, Bf16>(a, s) : launch_prefill_wide<128, Bf16>(a, s);
     return head_dim == 64 ? launch_prefill_wide<64, Fp16>(a, s) : launch_prefill_wide<128, Fp16>(a, s);
@@ -2930,6 +2948,17 @@ int prefill_impl(const void* q, void* out, const void* k_pool, const void* v_poo
 }
 
 }  // namespace
+
+extern "C" int fe_prefill_form(int num_seqs, int total_q, int max_q_len, int num_q_heads,
+                               int kv_heads, int head_dim, int block_size, int table_stride,
+                               int elem_bytes, int planned) {
+  FE_CHECK_ARG(num_seqs > 0 && total_q > 0 && max_q_len >= 0 && num_q_heads > 0 && kv_heads > 0 &&
+               head_dim > 0 && block_size > 0 && table_stride > 0 &&
+               (elem_bytes == 2 || elem_bytes == 4));
+  FE_CHECK_ARG(num_q_heads % kv_heads == 0);
+  return prefill_form(num_seqs, total_q, max_q_len, num_q_heads, kv_heads, head_dim, block_size,
+                      table_stride, elem_bytes == 4, planned != 0);
+}
 
 extern "C" int fe_prefill_paged(const void* q, void* out, const void* k_pool, const void* v_pool,
                                 int num_blocks, const int32_t* block_tables, int table_stride,

@@ -522,6 +522,20 @@ def plan_error(plan: DecodePlan | PrefillPlan) -> int:
     return int(plan.buffer[off:off + 4].view(torch.int32).item())
 
 
+_PREFILL_FORMS = ("generic", "tile", "stream", "wide", "f32")
+
+
+def prefill_form(num_seqs: int, total_q: int, max_q_len: int, num_q_heads: int, kv_heads: int,
+                 head_dim: int, block_size: int, table_stride: int, dtype: torch.dtype, *,
+                 planned: bool = False) -> str:
+    """The kernel that prefill_paged runs on at these sizes (fe_prefill_form)."""
+    rc = _lib.load().fe_prefill_form(num_seqs, total_q, max_q_len, num_q_heads, kv_heads, head_dim,
+                                     block_size, table_stride, dtype.itemsize, int(planned))
+    if rc < 0:
+        _lib.check("fe_prefill_form", rc)
+    return _PREFILL_FORMS[rc]
+
+
 def prefill_paged(q: torch.Tensor, k_pool: torch.Tensor, v_pool: torch.Tensor,
                   block_tables: torch.Tensor, q_offsets: torch.Tensor,
                   context_lens: torch.Tensor, max_q_len: int, *, scale: float | None = None,
@@ -531,7 +545,9 @@ def prefill_paged(q: torch.Tensor, k_pool: torch.Tensor, v_pool: torch.Tensor,
     q_offsets[s]:q_offsets[s+1] at positions context_lens[s]-n_s .. context_lens[s]-1.
     fp16, bf16 or float32 (q, out and the pools alike).  With `plan`
     (prefill_paged_plan on these q_offsets / context_lens and sizes; 16-bit pools)
-    the launch reads its work split from it (fe_prefill_paged_planned); same results."""
+    the launch reads its work split from it (fe_prefill_paged_planned); same results.
+    Tables no wider than the longest context let it choose the fastest kernel
+    (prefill_form): it takes the width for that length."""
     dev = _require_gpu(q, k_pool, v_pool, block_tables, q_offsets, context_lens, out)
     nb, bs, hkv, d = _check_pool(k_pool, v_pool, KV_DTYPES)
     if q.ndim != 3 or q.shape[2] != d or q.dtype != k_pool.dtype or not q.is_contiguous():

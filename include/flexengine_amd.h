@@ -540,6 +540,24 @@ int fe_prefill_paged_f32(const void* q, void* out,
                          void* workspace, size_t workspace_bytes, fe_stream_t stream);
 
 /*
+ * Which kernel a fe_prefill_paged call (elem_bytes 2, or 4 for the _f32 form;
+ * planned != 0: a _planned call) of these sizes runs on: FE_PREFILL_GENERIC
+ * (head dims without matrix-core kernels), _TILE (block sizes that are not
+ * multiples of 16, padded head dims, 256), _STREAM (stream-K key ranges),
+ * _WIDE (256-row blocks, long or fresh prompts) or _F32; a negative
+ * FE_ERR_* code for bad sizes.  The choice between _STREAM and _WIDE takes
+ * table_stride * block_size for the longest context.  Launches nothing; for
+ * tests and profiles.  No counterpart in the reference.
+ */
+#define FE_PREFILL_GENERIC 0
+#define FE_PREFILL_TILE 1
+#define FE_PREFILL_STREAM 2
+#define FE_PREFILL_WIDE 3
+#define FE_PREFILL_F32 4
+int fe_prefill_form(int num_seqs, int total_q, int max_q_len, int num_q_heads, int kv_heads,
+                    int head_dim, int block_size, int table_stride, int elem_bytes, int planned);
+
+/*
  * Prefill plan of one model step: the stream-K work split of fe_prefill_paged
  * -- every workgroup's range of key blocks and its first unit -- depends only
  * on q_offsets, context_lens and the sizes, which all layers of a step share.

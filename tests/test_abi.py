@@ -182,3 +182,25 @@ def test_plan_error_word_constants_match_the_header():
     assert int(macros["FE_PREFILL_PLAN_ERROR_OFFSET"]) == ops._PLAN_ERROR_OFFSET["PrefillPlan"]
     assert int(macros["FE_PLAN_ERR_SIZES"]) == ops.PLAN_ERR_SIZES
     assert int(macros["FE_PLAN_ERR_STALE"]) == ops.PLAN_ERR_STALE
+
+
+def test_prefill_form_chooses_by_sizes(lib):
+    """The kernel of a prefill from its sizes alone: block size, head dim and type first, then
+    the estimate that takes the table's width for the longest context."""
+    import torch
+
+    from flexengine_amd import ops
+
+    def form(n, cached=0, hq=12, hkv=2, d=128, bs=16, width=0, dtype=torch.float16, seqs=1):
+        w = width or -(-(n + cached) // bs)
+        return ops.prefill_form(seqs, n * seqs, n, hq, hkv, d, bs, w, dtype)
+    assert form(500) == form(8191, hq=32, hkv=8) == form(4096, hq=14, d=64) == "wide"
+    assert form(500, seqs=8) == "wide"
+    assert form(100, 1000) == form(16, 4000, hq=32, hkv=8) == form(1, 640, hq=14, d=64) == "stream"
+    assert form(8191, hq=32, hkv=8, width=2048) == "stream"       # four times the context
+    assert form(500, bs=8) == form(70, d=96) == form(70, d=256) == "tile"
+    assert form(70, d=260) == form(70, d=20) == form(70, d=256, dtype=torch.float32) == "generic"
+    assert form(70, dtype=torch.float32) == form(70, d=96, dtype=torch.float32) == "f32"
+    assert ops.prefill_form(1, 70, 70, 12, 2, 96, 16, 5, torch.float16, planned=True) == "generic"
+    assert lib.fe_prefill_form(1, 70, 70, 12, 5, 128, 16, 5, 2, 0) == _lib.FE_ERR_INVALID_ARGUMENT
+    assert lib.fe_prefill_form(0, 0, 0, 12, 2, 128, 16, 5, 2, 0) == _lib.FE_ERR_INVALID_ARGUMENT

@@ -36,6 +36,12 @@ def _case(seed, n_new, cached, hq=12, hkv=2, d=128, bs=16):
     return q, torch.tensor(offs), torch.tensor(ctx, dtype=torch.int32), tables, k_pool, v_pool
 
 
+def _form(q, k, t, new, planned=False):
+    """The kernel a prefill of these tensors runs on."""
+    return ops.prefill_form(len(new), q.shape[0], max(new), q.shape[1], k.shape[2], k.shape[3],
+                            k.shape[1], t.shape[1], q.dtype, planned=planned)
+
+
 def _run(q, offs, ctx, tables, kp, vp):
     n_new = (offs[1:] - offs[:-1]).tolist()
     out = ops.prefill_paged(q.to(DEV), kp.to(DEV), vp.to(DEV), tables.to(DEV), offs.to(DEV),
@@ -312,6 +318,7 @@ def test_prefill_rows_of_fresh_prompts_match_float64(dtype, max_tol, mean_tol, n
     o = torch.tensor(offs, dtype=torch.int32, device=DEV)
     c = torch.tensor(ctx, dtype=torch.int32, device=DEV)
     t = tables.to(DEV)
+    assert _form(q, k, t, new) == "wide"
     got = ops.prefill_paged(q, k, v, t, o, c, max(new))
     plan = ops.prefill_paged_plan(o, c, sum(new), hq, hkv, width, bs)
     assert torch.equal(ops.prefill_paged(q, k, v, t, o, c, max(new), plan=plan), got)
@@ -341,6 +348,7 @@ def test_wide_prefill_counts_probabilities_below_the_smallest_normal():
     t = torch.arange(n // bs, dtype=torch.int32, device=DEV)[None].contiguous()
     o = torch.tensor([0, n], dtype=torch.int32, device=DEV)
     c = torch.tensor([n], dtype=torch.int32, device=DEV)
+    assert _form(q, k, t, [n]) == "wide"
     got = ops.prefill_paged(q, k, v, t, o, c, n).double()
     top = float(q[0, 0, 0].double() * k[0, 0, 0, 0].double()) / d ** 0.5
     tail = torch.arange(n, device=DEV).double()[:, None, None] * math.exp(-top)
@@ -364,6 +372,7 @@ def test_wide_prefill_never_uses_rows_past_a_context(d, dtype):
     t = t.to(DEV)
     o = torch.tensor([0, new[0], sum(new)], dtype=torch.int32, device=DEV)
     c = torch.tensor(new, dtype=torch.int32, device=DEV)
+    assert _form(q, k, t, new) == "wide"
     good = ops.prefill_paged(q, k, v, t, o, c, max(new))
     for pool in (k, v):
         pool[sum(pages):] = float("nan")
@@ -383,6 +392,7 @@ def test_wide_prefill_refuses_a_stale_plan():
     t = torch.arange(pages, dtype=torch.int32, device=DEV)[None].contiguous()
     o = torch.tensor([0, n], dtype=torch.int32, device=DEV)
     c = torch.tensor([n], dtype=torch.int32, device=DEV)
+    assert _form(q, k, t, [n], planned=True) == "wide"
     plan = ops.prefill_paged_plan(o, c, n, hq, hkv, pages, bs)
     good = ops.prefill_paged(q, k, v, t, o, c, n, plan=plan)
     c.add_(1)
@@ -432,21 +442,22 @@ def _heads_float64(q, k, v, t, offs, ctx, heads):
             yield s, h, slice(offs[s], offs[s + 1]), sc.masked_fill_(causal, float("-inf")), vh
 
 
-@pytest.mark.parametrize("dtype,new,cached,hq,hkv,d,bs", [
-    (torch.bfloat16, [500], [0], 12, 2, 128, 16),            # wide: a fresh prompt
-    (torch.bfloat16, [64] * 6, [500] * 6, 12, 2, 128, 16),   # wide: chunks over cached tokens
-    (torch.float16, [100] * 16, [100] * 16, 14, 2, 64, 32),
-    (torch.float16, [100], [1000], 12, 2, 128, 16),          # stream-K, several blocks a range
-    (torch.bfloat16, [16], [4000], 32, 8, 128, 16),
-    (torch.float16, [90, 40], [3000, 2500], 14, 2, 64, 16),
+@pytest.mark.parametrize("form,dtype,new,cached,hq,hkv,d,bs", [
+    ("wide", torch.bfloat16, [500], [0], 12, 2, 128, 16),           # a fresh prompt
+    ("wide", torch.bfloat16, [64] * 6, [500] * 6, 12, 2, 128, 16),  # chunks over cached tokens
+    ("wide", torch.float16, [100] * 16, [100] * 16, 14, 2, 64, 32),
+    ("stream", torch.float16, [100], [1000], 12, 2, 128, 16),       # several blocks a range
+    ("stream", torch.bfloat16, [16], [4000], 32, 8, 128, 16),
+    ("stream", torch.float16, [90, 40], [3000, 2500], 14, 2, 64, 16),
 ])
-def test_prefill_rounds_probabilities_relative_to_each_blocks_own_maximum(dtype, new, cached, hq, hkv,
-                                                                        d, bs):
+def test_prefill_rounds_probabilities_relative_to_each_blocks_own_maximum(form, dtype, new, cached,
+                                                                        hq, hkv, d, bs):
     """The error against 64 bits is no larger than with the probabilities of every 64-key block
     rounded to 16 bits relative to that block's own maximum and all else exact.  (One maximum
     per row, the first block's, is 2.5-10% worse.)  The bound's 0.5%: fp32 scores and sums move
     a probability across a rounding boundary now and then."""
     q, k, v, t, o, c, offs, ctx = _device_case(new, cached, hq, hkv, d, bs, dtype, sum(new) + d)
+    assert _form(q, k, t, new) == form
     got = ops.prefill_paged(q, k, v, t, o, c, max(new)).double()
     err = emu = 0.0
     for _, h, rows, sc, vh in _heads_float64(q, k, v, t, offs, ctx, range(hq)):
@@ -466,11 +477,12 @@ def test_prefill_rounds_probabilities_relative_to_each_blocks_own_maximum(dtype,
 
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
-@pytest.mark.parametrize("new,cached", [([600], [0]), ([70], [1500])])   # wide; stream-K
-def test_prefill_follows_falling_and_rising_scores(dtype, new, cached):
+@pytest.mark.parametrize("form,new,cached", [("wide", [600], [0]), ("stream", [70], [1500])])
+def test_prefill_follows_falling_and_rising_scores(dtype, form, new, cached):
     """Block maxima that fall by 12 from block to block and then rise again: the reference of
     the probabilities follows them down no further than the sums allow, and back up."""
     q, k, v, t, o, c, offs, ctx = _device_case(new, cached, 12, 2, 128, 16, dtype, 5)
+    assert _form(q, k, t, new) == form
     x, pages = ctx[0], t[0].long()
     step = -12.0 * (torch.arange(x, device=DEV) // 64).float()
     step = torch.maximum(step, step.flip(0))                       # falls, then rises
@@ -518,12 +530,13 @@ def _range_rule(new, cached, hq, hkv, nwg_max=256):
     ([5, 0, 9], [9000, 7, 3001], 71, 1, 64, 16),
     ([1, 2], [640, 4000], 14, 2, 64, 16),            # too few rows: as with any length
     ([1] * 5, [2841] * 5, 28, 4, 128, 16),
-    ([37] * 70, [700] * 70, 12, 2, 128, 16),         # more blocks than three a workgroup
+    ([37] * 40, [3000] * 40, 12, 2, 128, 16),        # more blocks than three a workgroup
 ])
 def test_stream_k_ranges_follow_rows_and_blocks(dtype, max_tol, mean_tol, new, cached, hq, hkv, d, bs):
     """The split of chunks over cached tokens is the rule's, planned and unplanned give the
     same bits on one workspace call after call, and match float64."""
     q, k, v, t, o, c, offs, ctx = _device_case(new, cached, hq, hkv, d, bs, dtype, sum(cached))
+    assert _form(q, k, t, new) == _form(q, k, t, new, planned=True) == "stream"
     plan = ops.prefill_paged_plan(o, c, sum(new), hq, hkv, t.shape[1], bs)
     header = plan.buffer[:16].view(torch.int32).tolist()
     cus = torch.cuda.get_device_properties(0).multi_processor_count
@@ -536,3 +549,32 @@ def test_stream_k_ranges_follow_rows_and_blocks(dtype, max_tol, mean_tol, new, c
     for _, h, rows, sc, vh in _heads_float64(q, k, v, t, offs, ctx, sorted({0, hq // 2, hq - 1})):
         err = (got[rows, h].double() - torch.softmax(sc, -1) @ vh).abs()
         assert err.max() <= max_tol and err.mean() <= mean_tol, (h, err.max(), err.mean())
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("form,new,cached,hq,hkv,d,bs,q_scale", [
+    ("stream", [40, 130, 1], [3000, 200, 640], 12, 2, 128, 16, 8.0),
+    ("stream", [33, 129], [2990, 1], 14, 2, 64, 32, 16.0),
+    ("stream", [65, 1, 17], [2047, 63, 0], 16, 2, 128, 32, 1.0),
+    ("stream", [77], [1501], 14, 2, 64, 16, 1.0),
+    ("stream", [37] * 40, [3000] * 40, 12, 2, 128, 16, 8.0),
+    ("wide", [40, 130, 1], [300, 20, 64], 6, 1, 128, 16, 16.0),
+    ("wide", [900, 33], [0, 70], 14, 2, 64, 32, 16.0),
+])
+def test_prefill_large_scores_on_each_kernel(form, dtype, new, cached, hq, hkv, d, bs, q_scale):
+    """Scores over hundreds (q scaled), head groups of 7, 64-dim heads, blocks of 32 and odd
+    remainders, on the kernel named; a running maximum over part of a block's keys lets exp2
+    and the 16-bit probabilities overflow.  The bound: rounding of the output and, in the
+    numerator and the sum, of the probabilities, each half a unit of the 16-bit type; scores of
+    300 in fp32 move a probability by less than a hundredth of that in bf16, a tenth in fp16."""
+    q, k, v, t, o, c, offs, ctx = _device_case(new, cached, hq, hkv, d, bs, dtype, sum(new) + hq)
+    q = (q.float() * q_scale).to(dtype)
+    assert _form(q, k, t, new) == form
+    got = ops.prefill_paged(q, k, v, t, o, c, max(new))
+    plan = ops.prefill_paged_plan(o, c, sum(new), hq, hkv, t.shape[1], bs)
+    assert got.isfinite().all()
+    assert torch.equal(ops.prefill_paged(q, k, v, t, o, c, max(new), plan=plan), got)
+    unit = 2.0 ** (-11 if dtype == torch.float16 else -8)
+    for _, h, rows, sc, vh in _heads_float64(q, k, v, t, offs, ctx, sorted({0, hq // 2, hq - 1})):
+        err = (got[rows, h].double() - torch.softmax(sc, -1) @ vh).abs()
+        assert err.max() <= 3.2 * unit * vh.abs().max(), (h, err.max())
