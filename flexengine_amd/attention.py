@@ -49,9 +49,14 @@ def attention_for_request(q: torch.Tensor, cache, layer: int, request_id: str, l
     if length <= 0 or length > len(table_list) * cache.layout.block_size:
         raise ValueError("requested length is invalid/unreserved")
     scale = 1.0 / math.sqrt(q.shape[-1])
+    n = q.shape[0]
+    if n > 1:
+        # no more pages than the context has: the prefill takes what the table addresses for
+        # the longest context when it chooses its kernel
+        table_list = table_list[:-(-length // cache.layout.block_size)]
+    pages = len(table_list)
     # the table row, the length and the chunk's offsets in one copy to the device: three
     # small ones took 30 us a call, most of it host time, where the kernel takes 9
-    n, pages = q.shape[0], len(table_list)
     buf = torch.tensor([*table_list, length, 0, n], dtype=torch.int32).to(q.device,
                                                                         non_blocking=True)
     table, ctx, offs = buf.split((pages, 1, 2))

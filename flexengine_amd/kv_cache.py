@@ -399,17 +399,17 @@ class PagedKVCache:
         return torch.from_numpy(out).to(self.device, non_blocking=True)
 
     def device_tables(self, request_ids: Sequence[str | None], width: int | None = None,
-                      pad_block: int | None = None) -> torch.Tensor:
+                      pad_block: int | None = None, *, clip: bool = False) -> torch.Tensor:
         """block_table() gathered on the device from the device copy of the page
         tables (fe_gather_tables): the host sends one row index per request.  None
-        entries give rows of pad_block."""
+        entries give rows of pad_block.  clip: tables longer than width are cut there."""
         if self._dev is None:
             raise RuntimeError("device_tables needs a cache whose pools live on a GPU")
         live = [r for r in request_ids if r is not None]
         widest = max((self._pt.width_of(r) for r in live), default=1)
         if width is None:
             width = widest
-        elif widest > width:
+        elif widest > width and not clip:
             raise ValueError(f"a table has {widest} blocks, more than width {width}")
         rows = np.array([-1 if r is None else self._pt.row_of[r] for r in request_ids], np.int32)
         self._sync()

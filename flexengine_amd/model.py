@@ -172,8 +172,10 @@ class Qwen2Model:
             table = cache.tables[c.request_id]
             if any(cache.refs[table[p]] > 1 for p in range(c.start // bs, (end - 1) // bs + 1)):
                 raise RuntimeError("cannot write a shared immutable KV block")
-        width = max(len(cache.tables[c.request_id]) for c in chunks)
-        tables = cache.device_tables([c.request_id for c in chunks], width)
+        # the pages of the contexts, not those reserved ahead: the prefill takes what the
+        # tables address for the longest context when it chooses its kernel
+        width = max(-(-(c.start + len(c.input_ids)) // bs) for c in chunks)
+        tables = cache.device_tables([c.request_id for c in chunks], width, clip=True)
         q_offsets = torch.tensor([0] + [sum(lengths[:j + 1]) for j in range(len(lengths))],
                                  dtype=torch.int32).to(dev)
         ctx = torch.tensor([c.start + n for c, n in zip(chunks, lengths)], dtype=torch.int32).to(dev)

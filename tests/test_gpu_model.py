@@ -70,6 +70,21 @@ def test_forward_full_incremental_and_multi_request(d, hq, hkv):
     cache.assert_invariants()
 
 
+def test_pages_reserved_ahead_do_not_change_a_forward():
+    """Requests holding pages for tokens to come: the logits' bits are those of requests that
+    hold the chunk's pages only (the prefill chooses its kernel by the context)."""
+    model = tiny(128, 12, 2)
+    ids = [[(7 * i + j) % 320 for i in range(n)] for j, n in enumerate((700, 30))]
+    outs = []
+    for spare in (0, 6000):
+        cache = cache_for(model, 900, 16)
+        for j, x in enumerate(ids):
+            cache.reserve(f"r{j}", len(x) + spare)
+        outs.append(model.forward([Chunk(f"r{j}", x, 0) for j, x in enumerate(ids)], cache))
+    for got, want in zip(*outs):
+        assert torch.equal(got, want) and got.isfinite().all()
+
+
 def test_mixed_prefill_and_decode_chunks_in_one_forward():
     model = tiny()
     cache = cache_for(model)

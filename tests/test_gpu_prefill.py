@@ -578,3 +578,21 @@ def test_prefill_large_scores_on_each_kernel(form, dtype, new, cached, hq, hkv, 
     for _, h, rows, sc, vh in _heads_float64(q, k, v, t, offs, ctx, sorted({0, hq // 2, hq - 1})):
         err = (got[rows, h].double() - torch.softmax(sc, -1) @ vh).abs()
         assert err.max() <= 3.2 * unit * vh.abs().max(), (h, err.max())
+
+
+def test_pages_reserved_ahead_do_not_change_a_prefill():
+    """attention_for_request on a prompt whose request holds pages for later tokens: the
+    kernel, and so every bit, is that of a request holding the prompt's pages only."""
+    n, hq, hkv, d, bs = 1000, 12, 2, 128, 16
+    g = torch.Generator().manual_seed(91)
+    keys, values = (torch.randn(n, hkv, d, generator=g).half().to(DEV) for _ in range(2))
+    q = torch.randn(n, hq, d, generator=g).half().to(DEV)
+    outs = []
+    for reserved in (n, 8 * n):
+        cache = PagedKVCache(CacheLayout(1, 8 * n // bs, bs, hkv, d), device=DEV)
+        cache.reserve("r", reserved)
+        cache.write(0, "r", 0, keys, values)
+        outs.append(attention.attention_for_request(q, cache, 0, "r", n, torch.arange(n, device=DEV)))
+    assert torch.equal(outs[0], outs[1])
+    forms = [ops.prefill_form(1, n, n, hq, hkv, d, bs, w // bs, torch.float16) for w in (1008, 8 * n)]
+    assert forms == ["wide", "stream"]
