@@ -318,11 +318,24 @@ def test_f32_shared_prefix_with_page_write_and_long_prefix():
     plain = ops.paged_decode(d.q, d.k_pool, d.v_pool, d.block_tables, d.context_lens)
     close_f32(got, plain.cpu().numpy().astype(np.float64), "fp32 cascade vs plain")
 
-@pytest.mark.parametrize("hq,hkv,d", [(12, 2, 128), (14, 2, 64), (6, 2, 96)])
+
+@pytest.mark.parametrize("hq,hkv,d,bs", [(32, 8, 128, 16), (32, 4, 64, 32)])
+def test_f32_shared_prefix_of_many_rows(hq, hkv, d, bs):
+    """640 rows x 32 heads: the prefix pass runs two row tiles a workgroup (20480 rows), the
+    members' contexts ending inside the prefix, at its end and past it."""
+    lens = {3: 64, 100: 50, 639: 64 + 33, 7: 0}
+    w = to_f32(workloads.shared_prefix_workload(47 + d, [(640, 64)], singles=1, hq=hq, hkv=hkv, d=d,
+                                                block_size=bs, tail=(1, 40), member_lens=lens), 48)
+    got, _ = _shared_prefix(w)
+    exp, _, _ = oracle_decode(w)
+    close_f32(got, exp, f"fp32 cascade of 640 rows {hq}/{hkv}/{d}")
+
+
+@pytest.mark.parametrize("hq,hkv,d", [(12, 2, 128), (14, 2, 64), (6, 2, 96), (12, 2, 96), (16, 2, 40)])
 @pytest.mark.parametrize("new,cached", [
     ([1, 3, 16, 17], [0, 15, 16, 1]),       # fewer tiles than waves, row-tile edges
     ([64], [4100]),                         # a wave's tile list refilled (64 tiles of its own)
-    ([1900], [33]),                         # two row tiles a workgroup at 12 and 14 heads
+    ([1900], [33]),                         # two row tiles a workgroup from 12 heads on
 ])
 def test_f32_prefill_row_tile_forms(hq, hkv, d, new, cached):
     """One and two row tiles a workgroup, waves without tiles, and list and per-row table
