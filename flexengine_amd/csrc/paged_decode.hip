@@ -1610,9 +1610,11 @@ int decode_impl(const void* q, int64_t q_batch_stride, void* out, const void* k_
   // of 16k tokens): the piece kernel at the next of 64 / 128 / 256, the dims
   // past head_dim zeros in q and K and never stored
   // (fp32: the fp32 engine at 64 / 128, any block size; padded to 128 only when
-  // head_dim fills 3/4 of it.  Below that the padded form is faster as well -- D 80
-  // (32/8) 113 / 187 us at 64 rows of 128-4096 tokens, D 72 (16/2) 34 / 78 -- but the
-  // generic kernel takes contexts, block sizes and strides that it refuses)
+  // head_dim fills 3/4 of it.  The line was drawn where the engine, then at one wave per
+  // SIMD, lost to the generic kernel below; at two it wins at D 72 and 80 as well -- D 80
+  // (32/8) 113 / 187 us at 64 rows of 128-4096 tokens, D 72 (16/2) 34 / 78.  These stay
+  // on the generic kernel because it also takes contexts, block sizes and strides that the
+  // padded form refuses, which a rule that moved them would have to tell apart)
   const int dpad = mfma_padded_head_dim(head_dim);
   const bool padded = dpad != head_dim && plan == nullptr && cascade == nullptr &&
                       (f32 ? dpad == 64 || (dpad == 128 && 4 * head_dim >= 3 * dpad)

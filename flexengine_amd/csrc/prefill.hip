@@ -2309,8 +2309,9 @@ __device__ __forceinline__ void dma_block32(int kb, const unsigned char* kbase,
 // see more keys), so there are no partials, tickets or workspace; the dispatcher balances
 // them over the CUs.  K and V blocks come through a four-stage LDS-DMA ring (each wave
 // brings 8 keys of every block), three blocks in flight while one is computed.
-// 8191 tokens of 32/8 heads of 128 in bf16: 758 -> 516 us (725 -> 1064 TFLOP/s of the 1352
-// that a large matrix product reaches); of 14/2 heads of 64 in fp16 299 -> 163 us.
+// 8191 tokens of 32/8 heads of 128 in bf16, on the stream-K kernel / here: 764 / 520 us (720
+// / 1057 TFLOP/s, of the 1121-1352 that a large matrix product reaches); of 14/2 heads of 64
+// in fp16 298 / 167 us.
 constexpr int kWideRows = 256;
 constexpr int kWideRun = 8;      // keys of a block each wave brings in
 
@@ -2441,9 +2442,10 @@ void prefill_wide_kernel(const PrefillArgs a) {
     else if (j + 1 < nb) wait_vm<VM_BLOCK>();
     else wait_vm<0>();
     // a bare barrier: __syncthreads()'s release fence would also wait for the DMA of
-    // blocks j + 1 and j + 2.  The wait above has put this wave's run of block j in LDS;
-    // LDS operations of a wave complete in order, and the compiler fences keep every LDS
-    // access on its side of the barrier.
+    // blocks j + 1 and j + 2.  The wait above has put this wave's run of block j in LDS, and
+    // the compiler fences keep every LDS access on its side of the barrier.  Past it no wave
+    // reads block j - 1 any more, whose stage the DMA below fills: the MFMAs that consumed
+    // those reads were issued before it, each after the wait for its operands.
     asm volatile("" ::: "memory");
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
@@ -2596,11 +2598,11 @@ int launch_prefill_f32(PrefillArgs a, hipStream_t stream) {
 //     rounds of average ones;
 //   stream-K: 24 (ranges, partials, merge), 1.02 per key block of a workgroup's range, 4.5
 //     per unit in the first range (k units with cb cached blocks: k cb + k^2 / G blocks).
-// Measured, wide / stream-K, fp16, 12/2 heads of 128: fresh prompts of 500 20.6 / 28.8,
-// 1000 32.8 / 40.5, 2048 58.5 / 58.2, 4096 109 / 148, 8191 237 / 385, eight of 500 23 / 43;
-// over cached tokens 3 x 1000 + 2000 82 / 70, 4000 + 4000 201 / 163, four of 266-434 over
-// 1208-3012 89 / 41.  32/8 heads: 2048 fresh 61 / 105, 4 x 200 + 500 26 / 30, 1000 + 4000
-// 126 / 89.  14/2 of 64: 4096 fresh 80 / 112.
+// Measured, wide / stream-K, fp16, 12/2 heads of 128: fresh prompts of 500 21.3 / 28.9,
+// 1000 35.1 / 40.8, 2048 57.9 / 59.4, 4096 108 / 148, 8191 244 / 393, eight of 500 23 / 43;
+// over cached tokens 3 x 1000 + 2000 83 / 70, 4000 + 4000 207 / 169, four of 266-434 over
+// 1208-3012 92 / 45.  32/8 heads: 2048 fresh 62 / 105, 4 x 200 + 500 28 / 30, 1000 + 4000
+// 128 / 93.  14/2 of 64: 4096 fresh 81 / 112.
 inline bool use_wide(int num_seqs, int total_q, int max_q_len, int G, int kv_heads,
                      int64_t max_ctx, int cus) {
   const double ctx = (double)max_ctx;
