@@ -53,7 +53,7 @@ def attention_for_request(q: torch.Tensor, cache, layer: int, request_id: str, l
     if n > 1:
         # no more pages than the context has: the prefill takes what the table addresses for
         # the longest context when it chooses its kernel
-        table_list = table_list[:-(-length // cache.layout.block_size)]
+        table_list = table_list[:int(-(-length // cache.layout.block_size))]
     pages = len(table_list)
     # the table row, the length and the chunk's offsets in one copy to the device: three
     # small ones took 30 us a call, most of it host time, where the kernel takes 9

@@ -592,7 +592,10 @@ def test_pages_reserved_ahead_do_not_change_a_prefill():
         cache = PagedKVCache(CacheLayout(1, 8 * n // bs, bs, hkv, d), device=DEV)
         cache.reserve("r", reserved)
         cache.write(0, "r", 0, keys, values)
-        outs.append(attention.attention_for_request(q, cache, 0, "r", n, torch.arange(n, device=DEV)))
-    assert torch.equal(outs[0], outs[1])
+        # (a length may be any number that is whole)
+        for length in (n, float(n), torch.tensor(n)):
+            outs.append(attention.attention_for_request(q, cache, 0, "r", length,
+                                                        torch.arange(n, device=DEV)))
+    assert all(torch.equal(outs[0], x) for x in outs[1:])
     forms = [ops.prefill_form(1, n, n, hq, hkv, d, bs, w // bs, torch.float16) for w in (1008, 8 * n)]
     assert forms == ["wide", "stream"]
