@@ -319,6 +319,16 @@ def test_f32_shared_prefix_with_page_write_and_long_prefix():
     close_f32(got, plain.cpu().numpy().astype(np.float64), "fp32 cascade vs plain")
 
 
+@pytest.mark.parametrize("groups", [65, 260])
+def test_f32_shared_prefix_of_many_groups(groups):
+    """More groups than the prefix pass reads in one pass, and than in one round trip."""
+    w = to_f32(workloads.shared_prefix_workload(49, [(1 + i % 3, 16 * (i % 4)) for i in range(groups)],
+                                                singles=2, hq=6, hkv=2, d=64, tail=(1, 20)), 50)
+    got, _ = _shared_prefix(w)
+    exp, _, _ = oracle_decode(w)
+    close_f32(got, exp, f"fp32 cascade of {groups} groups")
+
+
 @pytest.mark.parametrize("hq,hkv,d,bs", [(32, 8, 128, 16), (32, 4, 64, 32)])
 def test_f32_shared_prefix_of_many_rows(hq, hkv, d, bs):
     """640 rows x 32 heads: the prefix pass runs two row tiles a workgroup (20480 rows), the

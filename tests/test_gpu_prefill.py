@@ -599,3 +599,20 @@ def test_pages_reserved_ahead_do_not_change_a_prefill():
     assert all(torch.equal(outs[0], x) for x in outs[1:])
     forms = [ops.prefill_form(1, n, n, hq, hkv, d, bs, w // bs, torch.float16) for w in (1008, 8 * n)]
     assert forms == ["wide", "stream"]
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("form,bs,hq,hkv,d", [("wide", 16, 12, 2, 128), ("tile", 8, 4, 4, 64)])
+@pytest.mark.parametrize("seqs", [64, 65, 256, 257, 300])
+def test_prefill_of_more_sequences_than_a_wave_holds(dtype, form, bs, hq, hkv, d, seqs):
+    """Row blocks are found among the sequences 64 at a time, four such passes a round trip past
+    64: sequences of no, one and a few tokens at the edges, against float64."""
+    new = [(0, 1, 5, 16, 3, 40)[i % 6] for i in range(seqs)]
+    new[-1] = 37
+    cached = [(0, 7, 33)[i % 3] for i in range(seqs)]
+    q, k, v, t, o, c, offs, ctx = _device_case(new, cached, hq, hkv, d, bs, dtype, seqs)
+    assert _form(q, k, t, new) == form
+    got = ops.prefill_paged(q, k, v, t, o, c, max(new)).double()
+    tol = 2e-3 if dtype == torch.float16 else 1.6e-2
+    for _, h, rows, sc, vh in _heads_float64(q, k, v, t, offs, ctx, (hq - 1,)):
+        assert (got[rows, h] - torch.softmax(sc, -1) @ vh).abs().max() <= tol, rows
